@@ -30,6 +30,7 @@ struct gs_context {
   int64_t exact_slot_bytes = 0;
   int32_t exact_slots = 0;
   int32_t cu_count = 0;  // compute units of the device (the scan's work split)
+  void* d_logprob = nullptr;  // partial sums of a tokenLogProbability call
   // constraint tables
   int64_t* d_vocab_offsets = nullptr;
   uint8_t* d_vocab_bytes = nullptr;
@@ -479,6 +480,7 @@ int gs_create(int device, int32_t vocab_size, int32_t max_rows, gs_context** out
     return cleanup(GS_ERR_HIP, "deep draw records");
   if (hipMalloc(&ctx->d_deep_queue, sizeof(DeepQueue) + sizeof(uint32_t) * 2 * (size_t)max_rows) != hipSuccess)
     return cleanup(GS_ERR_HIP, "deep draw queue");
+  if (hipMalloc(&ctx->d_logprob, logprob_bytes()) != hipSuccess) return cleanup(GS_ERR_HIP, "log-probability parts");
   *out = ctx;
   return GS_OK;
 }
@@ -493,6 +495,7 @@ int gs_destroy(gs_context* ctx) {
   free_dev(ctx->d_exact);
   free_dev(ctx->d_deep_rows);
   free_dev(ctx->d_deep_queue);
+  free_dev(ctx->d_logprob);
   free_dev(ctx->d_vocab_offsets);
   free_dev(ctx->d_vocab_bytes);
   free_dev(ctx->d_next);
@@ -744,7 +747,8 @@ int gs_token_log_prob(gs_context* ctx, const void* logits, int32_t dtype, int32_
   if (row_stride < ctx->vocab) return fail(ctx, GS_ERR_INVALID_ARGUMENT, "row_stride is smaller than the vocab");
   if (rows == 0) return GS_OK;
   GS_HIP(ctx, hipSetDevice(ctx->device));
-  launch_logprob(logits, dtype, rows, row_stride, ctx->vocab, tokens, out, pick_stream(ctx, stream));
+  launch_logprob(logits, dtype, rows, row_stride, ctx->vocab, tokens, out, ctx->d_logprob, ctx->cu_count,
+                 pick_stream(ctx, stream));
   GS_HIP(ctx, hipGetLastError());
   return GS_OK;
 }
@@ -770,7 +774,8 @@ int gs_token_log_prob_host(gs_context* ctx, const float* logits, int32_t rows, c
   hipStream_t s = ctx->stream;
   GS_HIP(ctx, hipMemcpyAsync(d, logits, logit_bytes, hipMemcpyHostToDevice, s));
   GS_HIP(ctx, hipMemcpyAsync(d + o_tok, tokens, sizeof(int32_t) * rows, hipMemcpyHostToDevice, s));
-  launch_logprob(d, GS_F32, rows, ctx->vocab, ctx->vocab, (const int32_t*)(d + o_tok), (double*)(d + o_out), s);
+  launch_logprob(d, GS_F32, rows, ctx->vocab, ctx->vocab, (const int32_t*)(d + o_tok), (double*)(d + o_out),
+                 ctx->d_logprob, ctx->cu_count, s);
   GS_HIP(ctx, hipGetLastError());
   GS_HIP(ctx, hipMemcpyAsync(out, d + o_out, sizeof(double) * rows, hipMemcpyDeviceToHost, s));
   GS_HIP(ctx, hipStreamSynchronize(s));
