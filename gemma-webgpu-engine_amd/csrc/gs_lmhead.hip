@@ -3,127 +3,271 @@
 //
 // The reference's producer is an int2 QAT GEMV (src/webgpu/decode-lm-head.ts:
 // 187-340); this is the bf16 tied-embedding variant the sampler consumes.
-// At M = 64 rows the product is bound by streaming W (2*V*D bytes) from HBM,
-// so the layout is built around W's reads:
-//   * a workgroup = 4 wave64, each wave owns 32 vocab rows; the grid covers V
-//     in slabs of 128 rows (and M in blocks of 64 rows);
-//   * per 64-wide K block a lane loads 64 contiguous bytes of one weight row
-//     (half the block: lanes 0-31 take k 0-31, lanes 32-63 take k 32-63), so
-//     each row's 128-byte line is consumed whole; weight and H loads run
-//     three K blocks ahead of their use in a register ring, so no wait
-//     covers a load issued less than two blocks earlier;
-//   * H's 64x64 block is staged in LDS (double-buffered, rows padded to 144 B)
-//     and shared by the four waves;
-//   * v_mfma_f32_32x32x16_bf16: a K block is 4 steps x 2 M tiles. The K order
-//     inside a block is permuted identically for H and W (step s, lane half h
-//     -> k = 32h + 8s + e), which leaves every dot product unchanged.
+// Two kernels, one order of sums: the K blocks of a row (64 wide) fall into
+// eight ranges, each summed by v_mfma_f32_16x16x32_bf16 in K order, and the
+// ranges are added one by one in binary32, so a logit is the same bits
+// whichever kernel and batch it comes from (and about half the rounding error
+// of one chain over K: 1.1e-7 against 2.0e-7 relative at D 2048).
+//   * up to 64 rows, widths up to 2048: lmhead_resident_kernel, H in registers;
+//   * anything else: lmhead_gemm_kernel, tiles of 128 vocabulary rows by up to
+//     128 rows of H. W is read from HBM once whatever M is (an XCD takes the
+//     row blocks of a slab of W one after another). At D 2048, V 262144:
+//     M 128 takes 220 us (5.5 TB/s), M 256 350, M 512 665 (830 TFLOP/s);
+//     the resident kernel, launched once per 64 rows, took 399, 793 and 1582.
+//     At M 12, D 3840, V 151643 217 us (5.4 TB/s) against 272 for a kernel
+//     that held the rows of W it multiplied in registers.
+// What bounds the GEMM: memory up to about 160 rows; past that the operand
+// traffic of the tiles (12 TB/s from the L2s at M 512), the matrix cores 42%
+// busy. The totals of the ranges take the registers that a larger tile would.
 #include "gs_internal.h"
 
 namespace gs {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kLmThreads = 256;
-constexpr int kLmRows = 128;  // vocab rows per workgroup
-constexpr int kLmM = 64;      // hidden rows per workgroup
-constexpr int kKBlock = 64;
-constexpr int kPad = 72;      // LDS row length in bf16 (64 + 8)
+// The K range (of eight) that the sums of vocabulary row v start with. Rows
+// of a multiple of 1024 bytes all start on the same few memory channels, and
+// every workgroup reads its rows' lines in the order of its sums: the slabs
+// of 128 rows start at different ranges, which spreads the chip's reads at
+// any time over the channels (M 128, D 2048, V 262144: 265 us with one start
+// for all, 230 so; widths off such strides measure the same either way).
+__device__ __forceinline__ int lmhead_first_range(int64_t v, int D) { return D % 512 == 0 ? (int)((v >> 7) & 7) : 0; }
 
-__device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
-
-__global__ __launch_bounds__(kLmThreads) void lmhead_kernel(const uint16_t* __restrict__ H,
-                                                            const uint16_t* __restrict__ W, int M, int D, int V,
-                                                            float cap, float* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][kLmM][kPad];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int h = lane >> 5;
-  const int n0 = blockIdx.x * kLmRows + wave * 32;
-  const int m0 = blockIdx.y * kLmM;
-  const int nrow = n0 + (lane & 31) < V ? n0 + (lane & 31) : V - 1;
-  const uint16_t* wrow = W + (size_t)nrow * D + h * 32;
-
-  // H: thread t stages 32 bytes of row t/4 of the 64x64 block (rows past M
-  // read row M-1 and are stored as zeros)
-  const int ar = tid >> 2, ac = (tid & 3) * 16;
-  const bool a_live = m0 + ar < M;
-  const uint16_t* hrow = H + (size_t)(a_live ? m0 + ar : M - 1) * D + ac;
-
-  // A ring of kDepth K-blocks in flight per lane: the weight row slice this
-  // lane multiplies (64 bytes) and this thread's share of the H block. The
-  // main loop is unrolled by kDepth and branch-free, so every ring slot is a
-  // fixed register set and each wait covers only loads issued kDepth - 1 or
-  // kDepth blocks earlier (loads complete in issue order). Prefetches past
-  // the last block re-read the last block (cache hits, never used).
-  constexpr int kDepth = 3;
-  const int nk = D / kKBlock;
-  uint4 wr[kDepth][4], hr[kDepth][2];
-  auto issue = [&](int slot, int kb) __attribute__((always_inline)) {
-    kb = kb < nk ? kb : nk - 1;
-    const uint4* pw = (const uint4*)(wrow + (size_t)kb * kKBlock);
-    const uint4* ph = (const uint4*)(hrow + (size_t)kb * kKBlock);
+// cap tanh(x / cap) of kN values of each lane. Below 5/8 tanh q is
+// q + q^3 P(q^2), P of degree 5 fitted over that range (relative error of the
+// fit 2^-32; at most 0.70 ulp with its roundings); a wave whose values all lie
+// there evaluates them side by side, where a tanhf a value, each behind its
+// own branch, was one long chain (60 of 690 us at M 512, D 2048, V 262144).
+// Their x / cap rounded to nearest takes two fused multiply-adds from
+// r = 1 / cap rounded to nearest (Markstein: the remainder of q0 = x r is
+// exact, and its share r completes the quotient). Every value takes the same
+// formula in either branch. r = 0 (cap outside 2^+-60): always the division.
+constexpr float kTanhSmall = 0.625f;
+__device__ __forceinline__ float tanh_small(float q) {
+  const float s = q * q;
+  float p = 0x1.197b58p-9f;
+  p = __builtin_fmaf(p, s, -0x1.0c213cp-7f);
+  p = __builtin_fmaf(p, s, 0x1.6394d6p-6f);
+  p = __builtin_fmaf(p, s, -0x1.b9ef7cp-5f);
+  p = __builtin_fmaf(p, s, 0x1.11106cp-3f);
+  p = __builtin_fmaf(p, s, -0x1.555554p-2f);
+  return __builtin_fmaf(q * s, p, q);
+}
+__device__ __forceinline__ float reciprocal_of_cap(float cap) {
+  return cap >= 0x1p-60f && cap <= 0x1p60f ? 1.0f / cap : 0.0f;
+}
+template <int kN>
+__device__ __forceinline__ void lmhead_cap(float (&x)[kN], float cap, float r) {
+  float q[kN];
+  bool small = r != 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wr[slot][i] = pw[i];
-    hr[slot][0] = ph[0];
-    hr[slot][1] = ph[1];
-  };
-  const uint32_t a_mask = a_live ? 0xFFFFFFFFu : 0u;  // rows past M stage zeros
-  auto stage_h = [&](int buf, int slot) __attribute__((always_inline)) {
-    const uint4 v0 = hr[slot][0], v1 = hr[slot][1];
-    *(uint4*)&sA[buf][ar][ac] = make_uint4(v0.x & a_mask, v0.y & a_mask, v0.z & a_mask, v0.w & a_mask);
-    *(uint4*)&sA[buf][ar][ac + 8] = make_uint4(v1.x & a_mask, v1.y & a_mask, v1.z & a_mask, v1.w & a_mask);
-  };
-
-  f32x16 acc0, acc1;
+  for (int e = 0; e < kN; ++e) {
+    const float q0 = x[e] * r;
+    q[e] = __builtin_fmaf(__builtin_fmaf(-q0, cap, x[e]), r, q0);
+    small = small && __builtin_fabsf(q[e]) < kTanhSmall;  // (false for a NaN)
+  }
+  if (__all(small)) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) { acc0[i] = 0.0f; acc1[i] = 0.0f; }
-  auto step = [&](int kbi, int p) __attribute__((always_inline)) {
-    const int buf = kbi & 1;
-    // the next block's H into the other buffer (its loads left kDepth-1 blocks ago)
-    stage_h(buf ^ 1, (p + 1) % kDepth);
+    for (int e = 0; e < kN; ++e) x[e] = cap * tanh_small(q[e]);
+  } else {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const bf16x8 bf = as_bf16x8(wr[p][s]);
-      const bf16x8 a0 = as_bf16x8(*(const uint4*)&sA[buf][lane & 31][h * 32 + s * 8]);
-      const bf16x8 a1 = as_bf16x8(*(const uint4*)&sA[buf][32 + (lane & 31)][h * 32 + s * 8]);
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, bf, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, bf, acc1, 0, 0, 0);
+    for (int e = 0; e < kN; ++e) {
+      const float v = x[e] / cap;
+      x[e] = cap * (__builtin_fabsf(v) < kTanhSmall ? tanh_small(v) : tanhf(v));
     }
-    issue(p, kbi + kDepth);  // refill this slot
-    __syncthreads();
-  };
+  }
+}
+
+constexpr int kGemmThreads = 256;  // 2 x 2 waves over (V, M)
+constexpr int kGemmV = 128;        // vocabulary rows per workgroup
+constexpr int kGemmK = 64;         // K block: one 128-byte line of every row
+constexpr int kGemmChunks = 8;     // K ranges summed one by one, as the resident kernel's waves do
+constexpr int kGemmStride = kGemmV + 4;  // LDS floats per staged output row
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* LdsPtr;
+
+// One K block's rows into LDS by the memory pipe alone (no registers): wave
+// instruction i of this wave takes 8 rows (lane / 8) of 128 bytes. Row r's
+// 16-byte chunk c lands at position c ^ (r & 7), so that the 8 lanes of an
+// operand read that go together hit 8 different 16-byte columns of the banks.
+template <int kInstr, typename Rsrc>
+__device__ __forceinline__ void gemm_fetch(Rsrc r, char* lds, const uint32_t (&off)[kInstr], uint32_t k) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass refuses the 16-byte size)
 #pragma unroll
-  for (int p = 0; p < kDepth; ++p) issue(p, p);
-  stage_h(0, 0);
+  for (int i = 0; i < kInstr; ++i)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (LdsPtr)(lds + 1024 * i), 16, off[i], k, 0, 0);
+#endif
+}
+
+// One K block: the next fetches go out, then two K-32 steps of this wave's
+// 4 x kMT tiles; `flush` (uniform) then moves the running tiles into the
+// totals. The buffers are distinct objects, so the compiler's own waits
+// before the reads cover nothing that is still being fetched.
+template <int kMT, typename Rsrc>
+__device__ __forceinline__ void gemm_block(const char* __restrict__ w, const char* __restrict__ h,
+                                           char* __restrict__ w_next, char* __restrict__ h_next,
+                                           Rsrc wr, Rsrc hr,
+                                           const uint32_t (&w_off)[4], const uint32_t (&h_off)[kMT], uint32_t w_k,
+                                           uint32_t h_k, const uint32_t (&pos)[2], bool flush,
+                                           f32x4 (&acc)[4][kMT], f32x4 (&total)[4][kMT]) {
+  gemm_fetch<kMT>(hr, h_next, h_off, h_k);
+  asm volatile("" ::: "memory");  // W's fetches stay the last four issued
+  gemm_fetch<4>(wr, w_next, w_off, w_k);
+  bf16x8 wf[2][4], hf[2][kMT];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) wf[s][a] = *(const bf16x8*)(w + pos[s] + 2048 * a);
+#pragma unroll
+    for (int b = 0; b < kMT; ++b) hf[s][b] = *(const bf16x8*)(h + pos[s] + 2048 * b);
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+#pragma unroll
+      for (int b = 0; b < kMT; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][a], hf[s][b], acc[a][b], 0, 0, 0);
+    }
+  }
+  if (flush) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+#pragma unroll
+      for (int b = 0; b < kMT; ++b) {
+        total[a][b] += acc[a][b];
+        acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
+  }
+}
+
+template <int kMT>  // 16-row tiles of H per wave: 32 kMT rows of H per workgroup
+__global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint16_t* __restrict__ H,
+                                                                      const uint16_t* __restrict__ W, int M, int D,
+                                                                      int V, int m_blocks, int wide, float cap,
+                                                                      float* __restrict__ out) {
+  constexpr int kRows = 32 * kMT;
+  constexpr int kWBytes = kGemmV * kGemmK * 2, kHBytes = kRows * kGemmK * 2;
+  // three blocks of W and two of H; the staged outputs take their place
+  __shared__ __attribute__((aligned(16))) char lds[3 * kWBytes + 2 * kHBytes];
+  static_assert(kRows * kGemmStride * 4 <= sizeof(lds), "the staged outputs fit where the operands were");
+  char *sw0 = lds, *sw1 = lds + kWBytes, *sw2 = lds + 2 * kWBytes, *sh0 = lds + 3 * kWBytes, *sh1 = sh0 + kHBytes;
+  // consecutive workgroups go to the XCDs in turn: an XCD takes the row
+  // blocks of one slab of W one after another, so W comes from HBM once and
+  // from that XCD's L2 for the other row blocks
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int vt = (local / m_blocks) * 8 + xcd;
+  const int64_t v0 = (int64_t)vt * kGemmV, m0 = (int64_t)(local % m_blocks) * kRows;
+  if (v0 >= V) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, g = lane >> 4, wv = wave & 1, wm = wave >> 1;
+  const int v_rows = V - v0 < kGemmV ? (int)(V - v0) : kGemmV;
+  const int m_rows = M - m0 < kRows ? (int)(M - m0) : kRows;
+  // rows past V or M read zeros
+  const __amdgpu_buffer_rsrc_t wr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(W + (size_t)v0 * D), (short)0, v_rows * D * 2, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t hr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(H + (size_t)m0 * D), (short)0, m_rows * D * 2, kBufferWord3);
+  // this wave fetches rows 32 wave .. + 31 of W's block and 8 kMT wave .. of H's
+  const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
+  uint32_t w_off[4], h_off[kMT];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w_off[i] = (uint32_t)((32 * wave + 8 * i + lr) * D * 2 + lc);
+#pragma unroll
+  for (int i = 0; i < kMT; ++i) h_off[i] = (uint32_t)((8 * kMT * wave + 8 * i + lr) * D * 2 + lc);
+  const int w_dst = 32 * wave * 128, h_dst = 8 * kMT * wave * 128;
+  // operand reads: lane (j, g) holds k = 32 s + 8 g .. + 7 of row j of a tile
+  uint32_t pos[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) pos[s] = (uint32_t)(j * 128 + (((4 * s + g) ^ (j & 7)) * 16));
+  const int w_src = 64 * wv * 128, h_src = 16 * kMT * wm * 128;
+
+  f32x4 acc[4][kMT], total[4][kMT];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+#pragma unroll
+    for (int b = 0; b < kMT; ++b) {
+      acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      total[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+  const int nk = D / kGemmK;
+  int range = 0, bound = 0;  // `bound`: the block that ends the current range (empty ranges are passed over)
+  auto next_bound = [&]() __attribute__((always_inline)) {
+    const int done = bound;
+    do { bound = ++range * nk / kGemmChunks; } while (bound == done && range < kGemmChunks);
+  };
+  next_bound();
+  const int first = lmhead_first_range(v0, D) * (nk / kGemmChunks);  // blocks wrap around after the last
+  auto at = [&](int kb) __attribute__((always_inline)) {
+    const int k = (kb < nk ? kb : nk - 1) + first;
+    return (uint32_t)((k < nk ? k : k - nk) * kGemmK * 2);
+  };
+  auto block = [&](int kb, char* w, char* h, char* wn, char* hn) __attribute__((always_inline)) {
+    // block kb's rows have landed for every wave (W's block kb + 1, fetched
+    // after them, may still be under way), and every wave has read block kb - 1
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const bool flush = kb + 1 == bound;
+    if (flush) next_bound();
+    gemm_block<kMT>(w + w_src, h + h_src, wn + w_dst, hn + h_dst, wr, hr, w_off, h_off, at(kb + 2), at(kb + 1), pos,
+                    flush, acc, total);
+  };
+  gemm_fetch<4>(wr, sw0 + w_dst, w_off, at(0));
+  gemm_fetch<kMT>(hr, sh0 + h_dst, h_off, at(0));
+  asm volatile("" ::: "memory");
+  gemm_fetch<4>(wr, sw1 + w_dst, w_off, at(1));
+  // blocks past the last are fetched as the last one again, and not read
+  for (int kb = 0;; kb += 6) {
+    block(kb, sw0, sh0, sw2, sh1);
+    if (kb + 1 >= nk) break;
+    block(kb + 1, sw1, sh1, sw0, sh0);
+    if (kb + 2 >= nk) break;
+    block(kb + 2, sw2, sh0, sw1, sh1);
+    if (kb + 3 >= nk) break;
+    block(kb + 3, sw0, sh1, sw2, sh0);
+    if (kb + 4 >= nk) break;
+    block(kb + 4, sw1, sh0, sw0, sh1);
+    if (kb + 5 >= nk) break;
+    block(kb + 5, sw2, sh1, sw1, sh0);
+    if (kb + 6 >= nk) break;
+  }
+  // nothing is in flight to or from LDS before the outputs take its place
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  // the cap, then the tile [m][v] through LDS, so that rows go out in pieces
+  // of 512 bytes (D layout: lane (j, g) holds column j, rows 4 g + e; the
+  // column is H's row, the rows are W's)
+  float* stage = (float*)lds;
+  const float rcap = reciprocal_of_cap(cap);
+#pragma unroll
+  for (int b = 0; b < kMT; ++b) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      float x[4] = {total[a][b][0], total[a][b][1], total[a][b][2], total[a][b][3]};
+      if (cap > 0.0f) lmhead_cap<4>(x, cap, rcap);
+      *(f32x4*)&stage[(16 * (kMT * wm + b) + j) * kGemmStride + 64 * wv + 16 * a + 4 * g] = f32x4{x[0], x[1], x[2], x[3]};
+    }
+  }
   __syncthreads();
-  const int n_main = nk - nk % kDepth;
-  for (int kb0 = 0; kb0 < n_main; kb0 += kDepth) {
-#pragma unroll
-    for (int p = 0; p < kDepth; ++p) step(kb0 + p, p);
-  }
-  // the last nk % kDepth blocks sit in the first ring slots
-#pragma unroll
-  for (int p = 0; p < kDepth - 1; ++p) {
-    if (n_main + p < nk) step(n_main + p, p);
-  }
-
-  // D layout of a 32x32 tile: lane l, register r -> column l % 32,
-  // row 8*(r/4) + 4*(l/32) + r%4
-  const int n = n0 + (lane & 31);
-  if (n >= V) return;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = 8 * (r >> 2) + 4 * h + (r & 3);
-    float x0 = acc0[r], x1 = acc1[r];
-    if (cap > 0.0f) {
-      x0 = cap * tanhf(x0 / cap);
-      x1 = cap * tanhf(x1 / cap);
+  float* o = out + (size_t)m0 * V + v0;
+  if (wide) {  // V % 4 == 0 and 16-byte aligned logits: a piece lies within its row
+#pragma unroll 4
+    for (int q = tid; q < kRows * kGemmV / 4; q += kGemmThreads) {
+      const int row = q / (kGemmV / 4), c = 4 * (q % (kGemmV / 4));
+      if (row < m_rows && c < v_rows)
+        __builtin_nontemporal_store(*(const f32x4*)&stage[row * kGemmStride + c], (f32x4*)&o[(size_t)row * V + c]);
     }
-    // non-temporal stores: the 64 x V logits stream past the caches (-11 us
-    // of 261 at M 64, D 2048, V 262144, against write-back stores)
-    if (m0 + row < M) __builtin_nontemporal_store(x0, &out[(size_t)(m0 + row) * V + n]);
-    if (m0 + 32 + row < M) __builtin_nontemporal_store(x1, &out[(size_t)(m0 + 32 + row) * V + n]);
+  } else {
+#pragma unroll 4
+    for (int q = tid; q < kRows * kGemmV; q += kGemmThreads) {
+      const int row = q / kGemmV, c = q % kGemmV;
+      if (row < m_rows && c < v_rows)
+        __builtin_nontemporal_store(stage[row * kGemmStride + c], &o[(size_t)row * V + c]);
+    }
   }
 }
 
@@ -133,15 +277,16 @@ __global__ __launch_bounds__(kLmThreads) void lmhead_kernel(const uint16_t* __re
 // D 2048) dealt round-robin to the workgroups, so the chip reads a window of
 // adjacent runs at a time (199 us against 203 us for one contiguous range
 // per workgroup).
-//   * 8 waves split K: wave w owns the 32-wide K steps [w nS / 8, (w+1) nS / 8)
-//     of the nS = D / 32, its H slice (64 rows) held as MFMA A operands
+//   * 8 waves split K: wave w owns the 64-wide K blocks [w nB / 8, (w+1) nB / 8)
+//     of the nB = D / 64, its H slice (64 rows) held as MFMA A operands
 //     (v_mfma_f32_16x16x32_bf16: lane i + 16 g holds k = 32 s + 8 g .. + 7 of
 //     row i of an M tile, 4 M tiles);
 //   * per step a lane loads 16 bytes per K step of one vocabulary row (the
 //     B operand), so the workgroup reads 16 whole rows of W (16 x 2D bytes,
 //     contiguous) per step; two steps of loads are in flight per wave;
 //   * the 8 waves' partial 64x16 tiles go through LDS (double-buffered), and
-//     after one barrier each thread adds two outputs' partials in wave order
+//     after one barrier each thread adds two outputs' partials in the order of
+//     their ranges (lmhead_first_range)
 //     and applies the cap into an LDS stage of 16 steps, which then goes out
 //     as 1 KB runs of each logits row in 16-byte stores. At M 64, D 2048,
 //     V 262144 the logits cost 73 us of 258 stored per step (64-byte pieces
@@ -153,6 +298,7 @@ __global__ __launch_bounds__(kLmThreads) void lmhead_kernel(const uint16_t* __re
 // take an out-of-range offset (zeros, no memory request; stores dropped). The
 // compiler's wait counts then cover exactly the loads a step consumes, as
 // loads and stores share one in-order counter on this part.
+constexpr int kResM = 64;         // hidden rows at most
 constexpr int kResWaves = 8;
 constexpr int kResThreads = 64 * kResWaves;
 constexpr int kResN = 16;         // vocabulary rows per step
@@ -162,10 +308,7 @@ constexpr int32_t kResNT = 2;     // non-temporal cache policy of the streams
 constexpr int kResStage = 16;     // steps of logits staged per flush
 constexpr int kResStageStride = kResStage * kResN + 4;  // LDS floats per staged row
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-template <int kS>  // K steps per wave, at most 8
+template <int kS>  // K steps per wave: 2, 4, 6 or 8
 __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint16_t* __restrict__ H,
                                                                       const uint16_t* __restrict__ W, int M, int D,
                                                                       int V, float cap, float* __restrict__ out) {
@@ -173,9 +316,9 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
   __shared__ __attribute__((aligned(16))) float stage[64 * kResStageStride];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 15, g = lane >> 4;
-  const int n_steps = D / 32;
-  const int s_lo = wave * n_steps / kResWaves, s_hi = (wave + 1) * n_steps / kResWaves;
-  const int my_steps = s_hi - s_lo;  // kS or kS - 1
+  const int n_blocks = D / 64;
+  const int s_lo = 2 * (wave * n_blocks / kResWaves), s_hi = 2 * ((wave + 1) * n_blocks / kResWaves);
+  const int my_steps = s_hi - s_lo;  // kS or kS - 2
   // this workgroup's steps k = 0 .. k_end - 1: run blockIdx.x + gridDim.x r
   // (r = k / kResStage), tile kResStage run + k % kResStage of 16 vocabulary
   // rows; steps on tiles past the last are empty
@@ -220,6 +363,7 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
       __builtin_amdgcn_make_buffer_rsrc((void*)out, (short)0, M * V * 4, kBufferWord3);
   // reduction role: outputs (m, n) = (2 (tid >> 4) + e, tid & 15), e = 0, 1
   const int rn = tid & 15, rm = 2 * (tid >> 4);
+  const float rcap = reciprocal_of_cap(cap);
   auto step = [&](int k, int u) __attribute__((always_inline)) {
     const int slot = u & 1;
     f32x4 acc[4];
@@ -237,19 +381,18 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) *(f32x4*)(r + 16 * mt) = acc[mt];
     __syncthreads();
-    float x0 = 0.0f, x1 = 0.0f;
+    const int first = lmhead_first_range((int64_t)tile_of(k) * kResN, D);
+    float x[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int w = 0; w < kResWaves; ++w) {
+    for (int i = 0; i < kResWaves; ++i) {
+      const int w = (first + i) & (kResWaves - 1);
       const float2 p = *(const float2*)&red[slot][w][rn * kResStride + rm];
-      x0 += p.x;
-      x1 += p.y;
+      x[0] += p.x;
+      x[1] += p.y;
     }
-    if (cap > 0.0f) {
-      x0 = cap * tanhf(x0 / cap);
-      x1 = cap * tanhf(x1 / cap);
-    }
-    stage[rm * kResStageStride + kResN * u + rn] = x0;
-    stage[(rm + 1) * kResStageStride + kResN * u + rn] = x1;
+    if (cap > 0.0f) lmhead_cap<2>(x, cap, rcap);
+    stage[rm * kResStageStride + kResN * u + rn] = x[0];
+    stage[(rm + 1) * kResStageStride + kResN * u + rn] = x[1];
   };
   // a staged run: piece q = tid + 512 i is 16 bytes of row q / 64 at column
   // 4 (q % 64), so a wave writes one row's 1 KB. Columns of tiles past the
@@ -289,38 +432,43 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
 
 void launch_lmhead(const uint16_t* hidden, const uint16_t* weight, int32_t m, int32_t width, int32_t vocab,
                    float softcap, float* out, int32_t cu_count, hipStream_t s, LaunchEvents ev) {
-  if (width <= kResMaxWidth && width % 32 == 0 && vocab % 4 == 0 && ((uintptr_t)out & 15) == 0 &&
-      (int64_t)vocab * kLmM * 4 < ((int64_t)1 << 31)) {
-    // one launch per 64-row block of H, one workgroup per compute unit
-    const int k_steps = (width / 32 + kResWaves - 1) / kResWaves;
+  if (width <= kResMaxWidth && width % 32 == 0 && m <= kResM && vocab % 4 == 0 && ((uintptr_t)out & 15) == 0 &&
+      (int64_t)vocab * kResM * 4 < ((int64_t)1 << 31)) {
+    // one workgroup per compute unit
+    const int k_steps = 2 * ((width / 64 + kResWaves - 1) / kResWaves);
     const dim3 grid(cu_count > 0 ? cu_count : 256), block(kResThreads);
-    for (int m0 = 0; m0 < m; m0 += kLmM) {
-      const int mb = m - m0 < kLmM ? m - m0 : kLmM;
-      const uint16_t* h = hidden + (size_t)m0 * width;
-      float* o = out + (size_t)m0 * vocab;
-      hipEvent_t start = m0 == 0 ? ev.start : nullptr, stop = m0 + kLmM >= m ? ev.stop : nullptr;
-      switch (k_steps) {
-#define GS_RES_CASE(k)                                                                                              \
-  case k:                                                                                                           \
-    hipExtLaunchKernelGGL(lmhead_resident_kernel<k>, grid, block, 0, s, start, stop, 0, h, weight, mb, width, vocab, \
-                          softcap, o);                                                                              \
+    switch (k_steps) {
+#define GS_RES_CASE(k)                                                                                               \
+  case k:                                                                                                            \
+    hipExtLaunchKernelGGL(lmhead_resident_kernel<k>, grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m,     \
+                          width, vocab, softcap, out);                                                               \
     break;
-        GS_RES_CASE(1)
-        GS_RES_CASE(2)
-        GS_RES_CASE(3)
-        GS_RES_CASE(4)
-        GS_RES_CASE(5)
-        GS_RES_CASE(6)
-        GS_RES_CASE(7)
-        GS_RES_CASE(8)
+      GS_RES_CASE(2)
+      GS_RES_CASE(4)
+      GS_RES_CASE(6)
+      GS_RES_CASE(8)
 #undef GS_RES_CASE
-      }
     }
     return;
   }
-  dim3 grid((vocab + kLmRows - 1) / kLmRows, (m + kLmM - 1) / kLmM);
-  hipExtLaunchKernelGGL(lmhead_kernel, grid, dim3(kLmThreads), 0, s, ev.start, ev.stop, 0, hidden, weight, m, width,
-                        vocab, softcap, out);
+  // blocks of at most 128 rows of H, the rows spread evenly over them
+  const int m_blocks = (m + 127) / 128;
+  const int tiles = ((m + m_blocks - 1) / m_blocks + 31) / 32;  // per wave: 1 .. 4
+  const int v_tiles = (vocab + kGemmV - 1) / kGemmV;
+  const dim3 grid((unsigned)((v_tiles + 7) / 8 * 8 * m_blocks)), block(kGemmThreads);
+  const int wide = vocab % 4 == 0 && ((uintptr_t)out & 15) == 0;
+  switch (tiles) {
+#define GS_GEMM_CASE(k)                                                                                               \
+  case k:                                                                                                             \
+    hipExtLaunchKernelGGL(lmhead_gemm_kernel<k>, grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m, width,   \
+                          vocab, m_blocks, wide, softcap, out);                                                       \
+    break;
+    GS_GEMM_CASE(1)
+    GS_GEMM_CASE(2)
+    GS_GEMM_CASE(3)
+    GS_GEMM_CASE(4)
+#undef GS_GEMM_CASE
+  }
 }
 
 }  // namespace gs

@@ -4,16 +4,15 @@
 // the reference's handoff this replaces is src/webgpu/decode-model.ts:127-150,
 // its producer src/webgpu/decode-lm-head.ts:262-340).
 //
-// Three launches replace lmhead_kernel + scan_kernel:
+// Three launches replace the lm_head and scan_kernel:
 //   * dead_bitmap_kernel, 16384 ids per workgroup: a row's excluded ids as a
 //     bitmap [rows][V/32] -- the ids its constraint mask forbids, its penalty
 //     window and its forced ids (the ids the scan leaves to the finish's exact
 //     evaluation) -- and the row's threshold word cleared;
-//   * lmhead_scan_kernel: the bf16 MFMA GEMM of lmhead_kernel over 256 vocab
-//     rows per workgroup (eight waves of one 32-row tile each, every wave with
-//     lmhead_kernel's register ring and per-lane K order, so the logits are
-//     bit-identical), the same softcap epilogue and
-//     non-temporal logits stores; then, per hidden row, the 256 logits of the
+//   * lmhead_scan_kernel: a bf16 MFMA GEMM over 256 vocab rows per workgroup
+//     (eight waves of one 32-row tile each: a lane holds the weight rows it
+//     multiplies in a register ring three K blocks deep, H goes through LDS),
+//     the softcap and non-temporal logits stores; then, per hidden row, the 256 logits of the
 //     workgroup's "partial" go through LDS into one statistics record and one
 //     candidate list, computed like a scan wave's: 16 lanes of 16 logits, the
 //     lane maxima, the normaliser in binary32 terms against each lane's maximum
@@ -257,7 +256,7 @@ __global__ __launch_bounds__(kFThreads, 2) void lmhead_scan_kernel(const uint16_
   const bool a_live = m0 + ar < M;
   const uint16_t* hrow = H + (size_t)(a_live ? m0 + ar : M - 1) * D + ac;
 
-  // lmhead_kernel's register ring: kDepth K blocks in flight, the loop
+  // the register ring: kDepth K blocks in flight, the loop
   // unrolled by kDepth and branch-free (prefetches past the last block
   // re-read it)
   const int nk = D / kFKBlock;
@@ -320,7 +319,7 @@ __global__ __launch_bounds__(kFThreads, 2) void lmhead_scan_kernel(const uint16_
   }
   // (the last step ended with a barrier: the H block is no longer read)
 
-  // softcap and the logits stores, as lmhead_kernel. D layout of a 32x32
+  // softcap and the logits stores. D layout of a 32x32
   // tile: lane l, register r -> column l % 32, row 8 (r / 4) + 4 (l / 32) + r % 4
   const int nl = lane & 31;
   const int n = n0 + nl;

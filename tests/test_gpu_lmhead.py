@@ -149,3 +149,45 @@ def test_lmhead_shapes_match_f64(vocab, width, m):
             assert bool((out[m:] == 7.0).all())
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("vocab,width,m,shift", [
+    (1000, 64, 65, 0),     # one K block, ranges without any; a partial slab
+    (4100, 448, 96, 0),    # fewer blocks than ranges; full three-tile row blocks
+    (4100, 512, 97, 0),    # ranges of one block, started in turn; the smallest four-tile block
+    (2052, 576, 129, 0),   # nine blocks over eight ranges; two row blocks
+    (1028, 1024, 257, 0),  # three row blocks
+    (4100, 2048, 128, 1),  # logits 4 bytes off a 16-byte address
+    (127, 2048, 33, 0),    # less than one slab, odd rows
+    (2049, 3840, 1, 0),    # wide, odd, one row
+])
+def test_lmhead_gemm_edges(vocab, width, m, shift):
+    """The tiled kernel at the edges of its tiles and ranges: against a float64 GEMM of every column,
+    and, where the resident kernel takes the first rows alone, equal to it bit for bit (both sum the
+    same ranges in the same order). Large logits as well, past the cap's small-argument polynomial."""
+    import torch
+
+    gs = _gs()
+    s = gs.Sampler(vocab_size=vocab, max_rows=8)
+    try:
+        dev = torch.device("cuda", 0)
+        hidden, weight = gs.workloads.lmhead_inputs(m, width, vocab, device=dev)
+        hidden = hidden.clone()
+        hidden[m // 2] *= 40  # logits well past the cap in one row
+        h, w = _f64(hidden), _f64(weight)
+        ref = h @ w.T
+        bound = GEMM_RTOL_OF_ABS_SUM * (np.abs(h) @ np.abs(w).T) + 1e-30
+        for cap in (0.0, 30.0):
+            store = torch.full(((m + 1) * vocab + shift,), 7.0, dtype=torch.float32, device=dev)
+            out = store[shift:].view(m + 1, vocab)
+            s.lmhead(hidden, weight, softcap_value=cap, out=out)
+            got = out[:m].cpu().numpy().astype(np.float64)
+            exp = cap * np.tanh(ref / cap) if cap > 0 else ref
+            err_bound = bound + (4 * np.spacing(np.abs(exp).astype(np.float32)).astype(np.float64) if cap > 0 else 0)
+            assert np.all(np.abs(got - exp) <= err_bound), (cap, float((np.abs(got - exp) / err_bound).max()))
+            assert bool((out[m:] == 7.0).all()) and bool((store[:shift] == 7.0).all())
+            if vocab % 4 == 0 and width <= 2048 and m > 64:
+                alone = s.lmhead(hidden[:64].contiguous(), weight, softcap_value=cap)
+                assert torch.equal(alone, out[:64])
+    finally:
+        s.close()
