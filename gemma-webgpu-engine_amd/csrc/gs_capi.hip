@@ -261,6 +261,7 @@ SampleArgs sample_args(const Workspace& w, const gs_batch* b) {
   a.deep_rows = deep ? w.deep_rows : nullptr;
   a.deep_queue = deep ? w.deep_queue : nullptr;
   a.deep_max_rows = deep ? w.deep_max_rows : 0;
+  a.typical = (b->hints & GS_BATCH_TYPICAL) != 0;
   return a;
 }
 
@@ -287,8 +288,14 @@ hipError_t launch_sample(const Workspace& w, const gs_batch* b, hipStream_t s, c
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
+  if (a.typical) {
+    // the typical-p rows that the finish left
+    launch_typical(a, s);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   if (b->rows > w.exact_slots) {
-    // rows past the slots were queued by the finish kernel
+    // rows past the slots were queued by the kernels before
     launch_exact(a, s, ev[GS_STAGE_EXACT]);
     e = hipGetLastError();
   }
@@ -661,6 +668,9 @@ int gs_sample_host(gs_context* ctx, const gs_batch* b, int32_t logits_on_device,
     const gs_row_config& c = b->configs[r];
     if (c.temperature > 0 && c.top_k <= 0 && c.top_p >= 1 && !(c.min_p > 0) && c.typical_p >= 1 && c.mask_slot < 0)
       db.hints |= GS_BATCH_FULL_DRAWS;
+    if (c.temperature > 0 && (c.top_k <= 0 || c.top_k >= ctx->vocab) && c.top_p >= 1 && !(c.min_p > 0) &&
+        c.typical_p < 1 && c.mask_slot < 0)
+      db.hints |= GS_BATCH_TYPICAL;
   }
   st = gs_sample(ctx, &db, s);
   if (st != GS_OK) return st;

@@ -4,12 +4,14 @@
 // 256-entry table and the quadratic 1 + r + r^2/2: relative error below
 // 4.2e-10 per evaluation (tests/test_scan_exp2.py pins it). exp2_256_tight
 // takes the quartic instead, for the deep draw's masses: relative error
-// below 1e-15 per evaluation.
+// below 1e-15 per evaluation. exp_neg is e^d within an ulp, for
+// log-probabilities and the typical-p rows.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include "gs_exp2_table.h"
+#include "gs_math.h"
 
 namespace gs {
 
@@ -39,6 +41,38 @@ __device__ __forceinline__ double exp2_256_tight(double y, const double* tab) {
   p = __builtin_fma(s, p, 1.0);
   const int ni = (int)n;
   return __builtin_ldexp(tab[ni & 255] * p, ni >> 8);
+}
+
+// exp_neg's factors 2^(j/32), one LDS bank pair each: random j never conflict
+constexpr int kExpTableBits = 5;
+constexpr int kExpTable = 1 << kExpTableBits;
+
+// e^d for d <= 0, within an ulp. Below -700 it is e^-700: a sum here is at
+// least 1, so no such term ever changes it.
+__device__ __forceinline__ double exp_neg(double d, const double* tab) {
+  constexpr double kInv = kExpTable * 1.44269504088896338700e+00;
+  constexpr double kHi = 6.93147180369123816490e-01 / kExpTable;  // 33 bits: k kHi is exact
+  constexpr double kLo = 1.90821492927058770002e-10 / kExpTable;
+  constexpr double kShift = 6755399441055744.0;  // 1.5 2^52: the sum's low word is the nearest integer
+  d = __builtin_fmax(d, -700.0);
+  const double z = __builtin_fma(d, kInv, kShift);
+  const double k = z - kShift;
+  const int i = (int)(uint32_t)gsm::bits_of(z);
+  const double r = __builtin_fma(-k, kLo, __builtin_fma(-k, kHi, d));
+  double p = __builtin_fma(r, 1.0 / 720.0, 1.0 / 120.0);
+  p = __builtin_fma(r, p, 1.0 / 24.0);
+  p = __builtin_fma(r, p, 1.0 / 6.0);
+  p = __builtin_fma(r, p, 0.5);
+  p = __builtin_fma(r, p, 1.0);
+  const double t = tab[i & (kExpTable - 1)];
+  // the exponent stays normal: i / kExpTable >= -1011
+  return gsm::double_of(gsm::bits_of(__builtin_fma(t * r, p, t)) + ((uint64_t)(uint32_t)(i >> kExpTableBits) << 52));
+}
+
+// (the whole workgroup calls it)
+__device__ __forceinline__ void load_exp_table(double* tab) {
+  if (threadIdx.x < kExpTable) tab[threadIdx.x] = c_exp2_256[threadIdx.x * (256 / kExpTable)];
+  __syncthreads();
 }
 
 }  // namespace gs

@@ -1341,6 +1341,7 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
     return 0;
   }
   if (plan.route == kRouteExact) {
+    if (a.typical && typical_row(a, row, cfg)) return 0;  // the typical-p kernel's
     return kExactRequest | 0u;
   }
   const bool greedy = plan.route == kRouteGreedy;

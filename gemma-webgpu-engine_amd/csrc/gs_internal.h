@@ -120,7 +120,8 @@ struct Plan {
 // deep, typical-p among them: its pool is the top-k); every other row keeps
 // 64 entries per chunk (top-p and min-p cuts, top-k up to kFinishCap, draws
 // over the whole vocabulary), and the finish resolves what falls inside the
-// complete region; typical-p over a longer pool, extreme temperatures and
+// complete region; typical-p over a longer pool (but for the typical-p kernel's
+// rows, which the finish leaves to it), extreme temperatures and
 // forced rows take the exact replay.
 __host__ __device__ __forceinline__ Plan plan_row(const gs_row_config& c) {
   if (c.temperature == 0) return Plan{kRouteGreedy, 1};
@@ -259,6 +260,7 @@ struct SampleArgs {
   DeepRow* deep_rows;      // [rows], or null: the finish's own workgroup takes its deep draws
   DeepQueue* deep_queue;
   int32_t deep_max_rows;   // pass-2 rows start at deep_queue->rows + deep_max_rows
+  int32_t typical;         // the typical-p kernel follows the finish and takes its rows
 };
 
 // Buffers of the fused lm_head + statistics path.
@@ -528,6 +530,17 @@ __device__ __forceinline__ void history_window(const SampleArgs& a, int64_t row,
   *end = h1;
 }
 
+// Rows of the typical-p kernel: typical-p alone over the whole vocabulary
+// (no penalties, mask, min-p, top-k or top-p), at temperatures where
+// div_by_temperature is the division.
+__device__ __forceinline__ bool typical_row(const SampleArgs& a, int64_t row, const gs_row_config& c) {
+  int64_t w0, w1;
+  history_window(a, row, c, &w0, &w1);
+  return c.typical_p > 0 && c.typical_p < 1 && (c.options & GS_ROW_FORCE_EXACT) == 0 &&
+         (c.top_k <= 0 || c.top_k >= a.vocab) && !(c.min_p > 0) && c.top_p >= 1 && c.mask_slot < 0 && w1 <= w0 &&
+         c.temperature >= 0x1p-20 && c.temperature <= 0x1p20;
+}
+
 // -------------------------------------------- distinct ids of one row
 // Hash of the row's distinct special ids (window ids with counts, forced
 // ids with kinds), built in LDS by one workgroup.
@@ -574,6 +587,7 @@ void launch_exp2_check(uint32_t first, uint32_t count, unsigned long long* worst
 void launch_finish(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
 void launch_exact(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
 void launch_deep(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
+void launch_typical(const SampleArgs& a, hipStream_t s);
 // partial: logprob_bytes() of device memory
 size_t logprob_bytes();
 void launch_logprob(const void* logits, int32_t dtype, int32_t rows, int64_t stride, int32_t vocab,

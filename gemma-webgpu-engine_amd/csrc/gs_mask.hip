@@ -77,8 +77,6 @@ __global__ __launch_bounds__(kMaskThreads) void build_masks_kernel(const int64_t
 // passes of 4-byte loads and fdlibm's exp took 297 us.
 constexpr int kLogThreads = 256;
 constexpr int kLogVecs = 4;  // 16-byte loads in flight per thread
-constexpr int kLogTableBits = 5;
-constexpr int kLogTable = 1 << kLogTableBits;
 constexpr int kLogParts = 2048;  // parts of a split call
 
 struct LogPart {
@@ -86,28 +84,6 @@ struct LogPart {
   float max;   // its maximum (-inf: no finite logit; NaN propagates)
   uint32_t pad;
 };
-
-// e^d for d <= 0, within an ulp. Below -700 it is e^-700: a sum here is at
-// least 1, so no such term ever changes it.
-__device__ __forceinline__ double exp_neg(double d, const double* tab) {
-  constexpr double kInv = kLogTable * 1.44269504088896338700e+00;
-  constexpr double kHi = 6.93147180369123816490e-01 / kLogTable;  // 33 bits: k kHi is exact
-  constexpr double kLo = 1.90821492927058770002e-10 / kLogTable;
-  constexpr double kShift = 6755399441055744.0;  // 1.5 2^52: the sum's low word is the nearest integer
-  d = __builtin_fmax(d, -700.0);
-  const double z = __builtin_fma(d, kInv, kShift);
-  const double k = z - kShift;
-  const int i = (int)(uint32_t)gsm::bits_of(z);
-  const double r = __builtin_fma(-k, kLo, __builtin_fma(-k, kHi, d));
-  double p = __builtin_fma(r, 1.0 / 720.0, 1.0 / 120.0);
-  p = __builtin_fma(r, p, 1.0 / 24.0);
-  p = __builtin_fma(r, p, 1.0 / 6.0);
-  p = __builtin_fma(r, p, 0.5);
-  p = __builtin_fma(r, p, 1.0);
-  const double t = tab[i & (kLogTable - 1)];
-  // the exponent stays normal: i / kLogTable >= -1011
-  return gsm::double_of(gsm::bits_of(__builtin_fma(t * r, p, t)) + ((uint64_t)(uint32_t)(i >> kLogTableBits) << 52));
-}
 
 // (m, s) joined with (om, os): both sums relative to the larger maximum. A
 // maximum of -inf has a sum of 0, one of NaN or +inf makes the sum NaN, as
@@ -138,11 +114,6 @@ __device__ __forceinline__ float logit_f32(In v) {
   else return v;
 }
 
-__device__ __forceinline__ void load_log_table(double* tab) {
-  if (threadIdx.x < kLogTable) tab[threadIdx.x] = c_exp2_256[threadIdx.x * (256 / kLogTable)];
-  __syncthreads();
-}
-
 // out for a row whose maximum and sum are known
 template <typename In>
 __device__ __forceinline__ double log_prob(const In* row, int32_t vocab, int32_t tok, float m, double s) {
@@ -157,10 +128,10 @@ __global__ __launch_bounds__(kLogThreads) void logprob_part_kernel(const In* log
                                                                    const int32_t* tokens, int32_t parts,
                                                                    LogPart* partial, double* out) {
   constexpr int kVec = 16 / (int)sizeof(In);
-  __shared__ double tab[kLogTable];
+  __shared__ double tab[kExpTable];
   __shared__ double s_sum[kLogThreads / 64];
   __shared__ float s_max[kLogThreads / 64];
-  load_log_table(tab);
+  load_exp_table(tab);
   const int64_t row = blockIdx.x / parts;
   const int part = (int)(blockIdx.x % parts);
   const In* base = logits + row * stride;
@@ -228,8 +199,8 @@ template <typename In>
 __global__ __launch_bounds__(kLogThreads) void logprob_join_kernel(const In* logits, int64_t stride, int32_t vocab,
                                                                    int32_t rows, const int32_t* tokens, int32_t parts,
                                                                    const LogPart* partial, double* out) {
-  __shared__ double tab[kLogTable];
-  load_log_table(tab);
+  __shared__ double tab[kExpTable];
+  load_exp_table(tab);
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * (kLogThreads / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;

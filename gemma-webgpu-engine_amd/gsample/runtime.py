@@ -27,6 +27,7 @@ GS_QAT_ROW_MAJOR, GS_QAT_BLOCK_MAJOR = 0, 1
 GS_RNG_SEEDED, GS_RNG_EXPLICIT = 0, 1
 GS_ROW_FORCE_EXACT = 1
 GS_BATCH_FULL_DRAWS = 1  # gs_batch.hints: a row may take a full-vocabulary draw
+GS_BATCH_TYPICAL = 4  # gs_batch.hints: a row may take typical-p over the whole vocabulary
 GS_BATCH_FUSED_HEAD = 2  # gs_batch.hints: gs_lmhead_sample computes the chunk statistics in the head
 GS_FORCED_TERMINATION, GS_FORCED_EXTRA = 1, 2
 GS_FLAG_TOPP_TIE = 1
@@ -248,6 +249,22 @@ def full_draw_rows(cfg: np.ndarray) -> bool:
                        & (c["typical_p"] >= 1) & (c["mask_slot"] < 0)))
 
 
+def batch_hints(cfg: np.ndarray, vocab: int) -> int:
+    """The hints of a batch of packed row configs: GS_BATCH_FULL_DRAWS as
+    full_draw_rows says, GS_BATCH_TYPICAL when a row may take typical-p over
+    the whole vocabulary (topK 0 or all, topP 1, no min-p, no mask)."""
+    c = np.asarray(cfg).reshape(-1)
+    if c.size == 1 and c["top_p"][0] < 1:  # an interactive row's usual options, settled by one field
+        return 0
+    free = (c["temperature"] > 0) & (c["top_p"] >= 1) & ~(c["min_p"] > 0) & (c["mask_slot"] < 0)
+    if not free.any():
+        return 0
+    typical, top_k = c["typical_p"] < 1, c["top_k"]
+    full = bool(np.any(free & ~typical & (top_k <= 0)))
+    spread = bool(np.any(free & typical & ((top_k <= 0) | (top_k >= vocab))))
+    return (GS_BATCH_FULL_DRAWS if full else 0) | (GS_BATCH_TYPICAL if spread else 0)
+
+
 def _csr(lists: Optional[Sequence[Sequence[int]]], rows: int):
     if lists is None:
         return None, None
@@ -315,7 +332,8 @@ class Sampler:
                 hints: Optional[int] = None):
         """Device-side batch for gs_sample; returns (Batch, keepalive). hints:
         the GS_BATCH_* bits, by default GS_BATCH_FULL_DRAWS when a row may take
-        a full-vocabulary draw."""
+        a full-vocabulary draw and GS_BATCH_TYPICAL when one may take typical-p
+        over the whole vocabulary."""
         torch = self.torch
         rows = int(logits.shape[0])
         if logits.dtype == torch.float32:
@@ -341,7 +359,7 @@ class Sampler:
         b.dtype = dtype
         b.rows = rows
         b.configs = d_cfg.data_ptr()
-        b.hints = (GS_BATCH_FULL_DRAWS if full_draw_rows(cfg) else 0) if hints is None else int(hints)
+        b.hints = batch_hints(cfg, int(logits.shape[1])) if hints is None else int(hints)
         if histories is not None:
             if isinstance(histories, tuple):
                 off, ids = histories

@@ -126,6 +126,13 @@ typedef struct gs_batch {
  * more than they save on average), those launches are skipped.
  * gs_sample_host sets the hint itself from its host configs. */
 #define GS_BATCH_FULL_DRAWS 1
+/* Batch hint: some row may take typical-p over the whole vocabulary
+ * (temperature > 0, topK 0 or the vocabulary's size, topP 1, no min-p, no
+ * mask). One more launch then settles such rows without penalties in one pass
+ * of exponentials (probabilities within 1e-14 relative), and replays exactly
+ * those whose decisions lie within the reference's rounding. Without the hint
+ * every such row is replayed. gs_sample_host sets the hint itself. */
+#define GS_BATCH_TYPICAL 4
 /* Batch hint for gs_lmhead_sample (vocabularies that are a multiple of 8192
  * ids): the lm_head's epilogue computes the chunk scan's statistics and
  * candidate lists itself, so the logits are written but not read back (three
