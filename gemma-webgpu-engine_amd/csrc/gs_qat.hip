@@ -370,6 +370,327 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
   }
 }
 
+// ---- the exact integer path for batches and for every width up to 2048
+//
+// Rows of x in groups of 16, a group's limbs resident in LDS for the whole
+// width: operand tile t holds the group's rows (kRows 16: limb t of each) or
+// limbs 2t and 2t + 1 of eight of them (kRows 8, where 16 rows' limbs would
+// not fit: more than 144 KB). A workgroup takes a run of 32-row vocabulary
+// pairs, a pair per wave: each code word is expanded once and multiplied by
+// every tile, and each limb tile read from LDS serves two vocabulary tiles
+// (64 lanes x 16 bytes per 32 cycles of a CU's matrix cores). Only as many
+// limbs are multiplied as the group's largest |A_k| has: 5 for activations of
+// an input SRQ, 5 or 6 for normal ones. The groups of one run are on one XCD,
+// so its codes come from HBM once.
+constexpr int kQatGemmThreads = 512;
+constexpr int kQatGemmWaves = kQatGemmThreads / 64;
+constexpr int kQatGroup = 16;
+constexpr int kQatMinTiles = 3;         // limb tiles multiplied at least
+constexpr int kQatOpBytes = 144 * 1024; // operand tiles in LDS
+
+struct QatGroupRows {
+  int emin[kQatGroup];                  // smallest granule exponent of the nonzero activations
+  uint32_t bad[kQatGroup];
+  unsigned long long sabs[kQatGroup];   // sum |A_k|
+  unsigned long long ssum[kQatGroup];   // sum A_k
+  uint32_t limbs;                       // of the group's largest |A_k|
+};
+
+union __attribute__((aligned(16))) QatGemmOp {
+  i32x4 op[kQatOpBytes / 16];  // [tile][step][lane]
+  float4 f[kQatGroup * 2048 / 4];  // the group's activations after the input SRQ, before
+  double act[2 * 2048];        // the binary64 path's activations
+};
+
+// The first `limbs` limbs of 16 activations, word W of row o of the group (row
+// o of eight for kRows 8), at their operand positions (see above).
+template <int kRows>
+__device__ __forceinline__ void qat_store_limbs(i32x4* op, int steps, int limbs, int o, int W, const int64_t (&A)[16]) {
+  constexpr uint64_t kK = 0x0080808080808080ull;
+  const int step = 4 * (W >> 4) + (W & 3), gw = (W >> 2) & 3;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint64_t u = ((uint64_t)A[4 * i + t] + kK) ^ kK;
+      lo[i] = (uint32_t)u;
+      hi[i] = (uint32_t)(u >> 32);
+    }
+#pragma unroll
+    for (int l = 0; l < 8; ++l) {
+      if (l >= limbs) break;
+      uint32_t dw = 0u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dw |= (((l < 4 ? lo[i] : hi[i]) >> (8 * (l & 3))) & 0xFFu) << (8 * i);
+      const int tile = kRows == 16 ? l : l >> 1, at = kRows == 16 ? o : 8 * (l & 1) + o;
+      ((uint32_t*)&op[(tile * steps + step) * 64 + at + 16 * gw])[t] = dw;
+    }
+  }
+}
+
+// Integers A_k = a_k / 2^E of 16 activations; false past the bound.
+__device__ __forceinline__ bool qat_integers(const float (&f)[16], int E, int64_t (&A)[16], uint64_t* sabs,
+                                             uint64_t* ssum, uint64_t* largest) {
+  bool ok = true;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    A[e] = 0;
+    uint32_t sig = 0;
+    int g = 0;
+    if (!act_parts(f[e], &sig, &g) || !sig) continue;
+    const int sh = g - E;
+    if (sh > 62 - 24) { ok = false; continue; }
+    const uint64_t mag = (uint64_t)sig << sh;
+    if (mag >= kQatSumBound) { ok = false; continue; }
+    A[e] = f[e] < 0.0f ? -(int64_t)mag : (int64_t)mag;
+    *sabs += mag;
+    *ssum += (uint64_t)A[e];
+    *largest = mag > *largest ? mag : *largest;
+  }
+  return ok;
+}
+
+// The run's vocabulary pairs [p_lo, p_hi) against rows r0 .. r0 + kRows - 1 of
+// the group at m0, its limbs in op.
+template <int kTiles, int kRows>
+__device__ __forceinline__ void qat_gemm_run(const QatArgs& a, const QatGroupRows& R, const i32x4* op, int m0, int r0,
+                                             int rows_here, uint32_t ok_rows, int p_lo, int p_hi, bool cached) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+  const int D = a.D, words = D / 16, blocks = D / 64, quads = (D + 255) / 256, steps = 4 * quads;
+  const __amdgpu_buffer_rsrc_t cr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.words, (short)0, a.V * words * 4, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, (short)0, a.V * 4, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.out + (int64_t)m0 * a.V), (short)0,
+                                                                       rows_here * a.V * 4, kBufferWord3);
+  constexpr int kQuads = kQatMaxSteps / 4;
+  u32x4 cw[2][kQuads];
+  // block 4 q + g of vocabulary row n; rows past V, blocks past the width and
+  // pairs past the run read zeros without a request
+  auto fetch = [&](int p, int v, int q) __attribute__((always_inline)) {
+    const uint32_t n = (uint32_t)p * 32u + (uint32_t)(16 * v + j);
+    const bool live = p < p_hi && n < (uint32_t)a.V && 4 * q + g < blocks;
+    const uint32_t off = a.block_major ? ((uint32_t)(4 * q + g) * (uint32_t)a.V + n) * 16u
+                                       : (n * (uint32_t)words + (uint32_t)(16 * q + 4 * g)) * 4u;
+    cw[v][q] = cached ? __builtin_amdgcn_raw_buffer_load_b128(cr, live ? off : kBufferOutOfRange, 0, 0)
+                      : __builtin_amdgcn_raw_buffer_load_b128(cr, live ? off : kBufferOutOfRange, 0, kQatNT);
+  };
+  // no branch around a load (see above): quads past the width read zeros
+  int p = p_lo + wave;
+#pragma unroll
+  for (int q = 0; q < kQuads; ++q) { fetch(p, 0, q); fetch(p, 1, q); }
+  // a step's limbs are read while the step before multiplies
+  i32x4 limb[2][kTiles];
+  auto read = [&](int step, i32x4 (&d)[kTiles]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) d[t] = op[(t * steps + step) * 64 + lane];
+  };
+  read(0, limb[0]);
+  for (; p < p_hi; p += kQatGemmWaves) {
+    const uint32_t n0 = (uint32_t)p * 32u + (uint32_t)j;
+    float sc[2];
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      sc[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                            sr, n0 + 16u * v < (uint32_t)a.V ? (n0 + 16u * v) * 4u : kBufferOutOfRange, 0, 0));
+    i32x4 acc[kTiles][2];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) acc[t][0] = acc[t][1] = i32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q) {
+      const uint32_t w0[4] = {cw[0][q].x, cw[0][q].y, cw[0][q].z, cw[0][q].w};
+      const uint32_t w1[4] = {cw[1][q].x, cw[1][q].y, cw[1][q].z, cw[1][q].w};
+      if (q < quads) {
+#pragma unroll
+        for (int tp = 0; tp < 4; ++tp) {
+          const int step = 4 * q + tp;
+          read(step + 1 < steps ? step + 1 : 0, limb[(tp + 1) & 1]);
+          constexpr uint32_t kLow = 0x03030303u;
+          const uint32_t x = w0[tp], y = w1[tp];
+          const i32x4 b0 = {(int)(x & kLow), (int)((x >> 2) & kLow), (int)((x >> 4) & kLow), (int)((x >> 6) & kLow)};
+          const i32x4 b1 = {(int)(y & kLow), (int)((y >> 2) & kLow), (int)((y >> 4) & kLow), (int)((y >> 6) & kLow)};
+#pragma unroll
+          for (int t = 0; t < kTiles; ++t) {
+            acc[t][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(limb[tp & 1][t], b0, acc[t][0], 0, 0, 0);
+            acc[t][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(limb[tp & 1][t], b1, acc[t][1], 0, 0, 0);
+          }
+          // (the limb reads of later steps hoisted over these spill registers)
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      // the next pair's codes into the registers these leave
+      fetch(p + kQatGemmWaves, 0, q);
+      fetch(p + kQatGemmWaves, 1, q);
+    }
+    // lane (j, g) holds rows 4 g .. 4 g + 3 of every tile; the limbs combine
+    // in wrapping 64-bit arithmetic (the totals are below 2^53)
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint64_t s = 0;
+        if constexpr (kRows == 16) {
+#pragma unroll
+          for (int t = 0; t < kTiles; ++t) s += (uint64_t)(int64_t)acc[t][v][e] << (8 * t);
+        } else {
+#pragma unroll
+          for (int t = 0; t < kTiles; ++t) s += (uint64_t)(int64_t)acc[t][v][e] << (8 * (2 * t + (g >> 1)));
+          s += shfl_xor_u64(s, 32);
+        }
+        const int r = r0 + (kRows == 16 ? 4 * g + e : 4 * (g & 1) + e);
+        const int64_t T = (int64_t)(s - 2 * (uint64_t)R.ssum[r]);
+        const double dot = __builtin_ldexp((double)T, R.emin[r] != 0x7FFFFFFF ? R.emin[r] : 0);
+        const float y = (float)srq(dot * (double)sc[v], a.out_scale);
+        const uint32_t n = n0 + 16u * v;
+        const bool st = (ok_rows >> r & 1u) != 0 && n < (uint32_t)a.V && (kRows == 16 || g < 2);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), orr,
+                                              st ? ((uint32_t)r * (uint32_t)a.V + n) * 4u : kBufferOutOfRange, 0, 0);
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kQatGemmThreads) void qat_gemm_kernel(QatArgs a, int32_t n_groups, int32_t n_runs) {
+  __shared__ QatGemmOp L;
+  __shared__ QatGroupRows R;
+  const int tid = threadIdx.x;
+  const int D = a.D, words = D / 16, quads = (D + 255) / 256, steps = 4 * quads;
+  // runs 8 i .. 8 i + 7 of every group follow each other: run k is on XCD k % 8
+  const int band = blockIdx.x / (8 * n_groups), in_band = blockIdx.x % (8 * n_groups);
+  const int group = in_band / 8, run = 8 * band + in_band % 8;
+  if (run >= n_runs) return;
+  const int m0 = kQatGroup * group;
+  const int rows_here = a.M - m0 < kQatGroup ? a.M - m0 : kQatGroup;
+  const int n_pairs = (a.V + 31) / 32;
+  const int p_lo = (int)((int64_t)run * n_pairs / n_runs), p_hi = (int)((int64_t)(run + 1) * n_pairs / n_runs);
+  if (tid < kQatGroup) { R.emin[tid] = 0x7FFFFFFF; R.bad[tid] = 0; R.sabs[tid] = 0; R.ssum[tid] = 0; }
+  if (tid == 0) R.limbs = 0;
+  __syncthreads();
+  // the group's activations, after the input SRQ, by words of 16: thread t
+  // takes words t, t + kQatGemmThreads, ..
+  const float4* x = (const float4*)(a.x + (int64_t)m0 * D);
+  const int n_words = rows_here * words;
+#pragma unroll 1
+  for (int k = tid; k < n_words; k += kQatGemmThreads) {
+    int gmin = 0x7FFFFFFF;
+    bool bad = false;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float4 q = x[4 * k + v];
+      float e[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        e[i] = (float)srq((double)e[i], a.in_scale);
+        uint32_t sig;
+        int g;
+        if (!act_parts(e[i], &sig, &g)) bad = true;
+        else if (sig) gmin = g < gmin ? g : gmin;
+      }
+      L.f[4 * k + v] = make_float4(e[0], e[1], e[2], e[3]);
+    }
+    if (gmin != 0x7FFFFFFF) atomicMin(&R.emin[k / words], gmin);
+    if (bad) atomicOr(&R.bad[k / words], 1u);
+  }
+  auto activations = [&](int k, float (&f)[16]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float4 q = L.f[4 * k + v];
+      f[4 * v] = q.x; f[4 * v + 1] = q.y; f[4 * v + 2] = q.z; f[4 * v + 3] = q.w;
+    }
+  };
+  __syncthreads();
+  uint64_t largest = 0;
+#pragma unroll 1
+  for (int k = tid; k < n_words; k += kQatGemmThreads) {
+    const int o = k / words;
+    float f[16];
+    activations(k, f);
+    int64_t A[16];
+    uint64_t sabs = 0, ssum = 0, big = 0;
+    const bool ok = qat_integers(f, R.emin[o] != 0x7FFFFFFF ? R.emin[o] : 0, A, &sabs, &ssum, &big);
+    atomicAdd(&R.sabs[o], (unsigned long long)sabs);
+    atomicAdd(&R.ssum[o], (unsigned long long)ssum);
+    if (!ok) atomicOr(&R.bad[o], 1u);
+    largest = big > largest ? big : largest;
+  }
+  {
+    // n limbs hold |A| up to 0x7F7F .. 7F (n bytes)
+    uint32_t limbs = 1;
+#pragma unroll
+    for (int n = 1; n < kQatLimbs; ++n) limbs += largest > (0x007F7F7F7F7F7F7Full >> (8 * (kQatLimbs - n))) ? 1u : 0u;
+    limbs = wave_max_u32(limbs);
+    if ((tid & 63) == 0) atomicMax(&R.limbs, limbs);
+  }
+  __syncthreads();
+  uint32_t ok_rows = 0;
+  for (int o = 0; o < rows_here; ++o) ok_rows |= !R.bad[o] && R.sabs[o] < kQatSumBound ? 1u << o : 0u;
+  const int limbs = (int)R.limbs < kQatMinTiles ? kQatMinTiles : (int)R.limbs;
+  const bool cached = n_groups > 1;
+
+  // The limbs take the activations' place in LDS, so these are read again.
+  // (Limbs of a refused row reach only outputs that are not stored.)
+  auto word = [&](int k, int64_t (&A)[16]) __attribute__((always_inline)) {
+    float e[16];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float4 q = x[4 * k + v];
+      e[4 * v] = (float)srq((double)q.x, a.in_scale);
+      e[4 * v + 1] = (float)srq((double)q.y, a.in_scale);
+      e[4 * v + 2] = (float)srq((double)q.z, a.in_scale);
+      e[4 * v + 3] = (float)srq((double)q.w, a.in_scale);
+    }
+    uint64_t u0 = 0, u1 = 0, u2 = 0;
+    const int E = R.emin[k / words];
+    (void)qat_integers(e, E != 0x7FFFFFFF ? E : 0, A, &u0, &u1, &u2);
+  };
+  if (ok_rows == 0) {
+    // nothing for the integer path
+  } else if (limbs * steps * 1024 <= kQatOpBytes) {
+    __syncthreads();
+#pragma unroll 1
+    for (int k = tid; k < n_words; k += kQatGemmThreads) {
+      int64_t A[16];
+      word(k, A);
+      qat_store_limbs<16>(L.op, steps, limbs, k / words, k % words, A);
+    }
+    __syncthreads();
+    switch (limbs) {
+      case 3: qat_gemm_run<3, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+      case 4: qat_gemm_run<4, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+      case 5: qat_gemm_run<5, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+      case 6: qat_gemm_run<6, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+      default: qat_gemm_run<7, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+    }
+  } else {
+    // eight rows at a time, all limbs (4 tiles: 128 KB at width 2048)
+#pragma unroll 1
+    for (int r0 = 0; r0 < rows_here; r0 += 8) {
+      __syncthreads();
+#pragma unroll 1
+      for (int k = tid; k < n_words; k += kQatGemmThreads) {
+        const int o = k / words;
+        if (o < r0 || o >= r0 + 8) continue;
+        int64_t A[16];
+        word(k, A);
+        qat_store_limbs<8>(L.op, steps, 8, o - r0, k % words, A);
+      }
+      __syncthreads();
+      qat_gemm_run<4, 8>(a, R, L.op, m0, r0, rows_here, ok_rows, p_lo, p_hi, cached);
+    }
+  }
+  // rows the check refused: the binary64 path over this run's vocabulary rows
+  for (int r0 = 0; r0 < rows_here; r0 += 2) {
+    const uint32_t two = rows_here - r0 >= 2 ? 3u : 1u, ok = ok_rows >> r0 & two;
+    if (ok == two) continue;
+    const bool skip[2] = {(ok & 1u) != 0, (ok & 2u) != 0};
+    __syncthreads();
+    qat_stage_act<2, kQatGemmThreads>(a, m0 + r0, L.act);
+    const int64_t end = (int64_t)p_hi * 32 < a.V ? (int64_t)p_hi * 32 : a.V;
+    for (int64_t r = (int64_t)p_lo * 32 + tid; r < end; r += kQatGemmThreads)
+      qat_row_binary64<2>(a, m0 + r0, skip, L.act, r);
+  }
+}
+
 }  // namespace
 
 // rows of x per pass for width D (the LDS stage holds kQatLdsDoubles)
@@ -383,13 +704,20 @@ void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* wor
                        const float* scales, int32_t V, double in_scale, double out_scale, float* out,
                        int32_t cu_count, hipStream_t s, LaunchEvents ev) {
   QatArgs a{x, words, scales, out, D, V, M, block_major, in_scale, out_scale};
-  if (D % 256 == 0 && D <= 2048 && V % 16 == 0) {
-    // one launch per pair of rows, one workgroup per compute unit
-    const int tiles = (M + 1) / 2;
-    for (int t = 0; t < tiles; ++t) {
-      hipExtLaunchKernelGGL(qat_tile_kernel, dim3(cu_count > 0 ? cu_count : 256), dim3(kQatTileThreads), 0, s,
-                            t == 0 ? ev.start : nullptr, t == tiles - 1 ? ev.stop : nullptr, 0, a, t);
-    }
+  const int cus = cu_count > 0 ? cu_count : 256;
+  if (D % 256 == 0 && D <= 2048 && V % 16 == 0 && M <= 2) {
+    // one or two rows: one workgroup per compute unit
+    hipExtLaunchKernelGGL(qat_tile_kernel, dim3(cus), dim3(kQatTileThreads), 0, s, ev.start, ev.stop, 0, a, 0);
+    return;
+  }
+  if (D <= 2048) {
+    // groups of 16 rows, about one workgroup per compute unit in all
+    const int groups = (M + kQatGroup - 1) / kQatGroup;
+    const int pairs = (V + 31) / 32;
+    int runs = cus / groups;
+    runs = runs < 1 ? 1 : (runs > pairs ? pairs : runs);
+    hipExtLaunchKernelGGL(qat_gemm_kernel, dim3(((runs + 7) / 8) * 8 * groups), dim3(kQatGemmThreads), 0, s, ev.start,
+                          ev.stop, 0, a, groups, runs);
     return;
   }
   const dim3 grid((unsigned)((V + kQatThreads - 1) / kQatThreads));

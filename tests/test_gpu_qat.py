@@ -170,3 +170,44 @@ def test_signed_zero_logits():
                 assert bad[0].size == 0, (in_s, out_s, layout, bad[0][:5], bad[1][:5], got[bad][:5], want[bad][:5])
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("V,D,M", [(1000, 64, 1), (1003, 320, 2), (96, 256, 3), (1000, 1536, 16), (2081, 1536, 17),
+                                   (515, 1984, 5), (1056, 2048, 9), (300, 2048, 35), (300, 2112, 3)])
+@pytest.mark.parametrize("in_scale", [0.0, 0.03])
+def test_row_groups_bit_exact(V, D, M, in_scale):
+    """Groups of 16 rows at every edge: vocabularies and widths that no tile
+    divides, last groups of one row, groups whose limbs fill LDS whole or
+    eight rows at a time (width 2048 with a wide exponent range), rows of few
+    limbs (small integers), zero rows, and rows only binary64 settles."""
+    import torch
+
+    gs = _gs()
+    rng = np.random.default_rng(V + D + M)
+    words = oracle.pack_int2_rows(rng.integers(0, 4, V * D, dtype=np.uint8), V, D)
+    scales = rng.uniform(0.0005, 0.005, V).astype(np.float32)
+    in_scale = float(np.float32(in_scale))
+    normal = rng.normal(0, 1.5, (M, D))
+    wide = normal * np.exp2(rng.integers(-18, 1, (M, D)))
+    integers = rng.integers(-60, 60, (M, D)).astype(np.float64)
+    mixed = np.where(np.arange(M)[:, None] % 3 == 0, wide, normal)
+    mixed[M // 2] = 0.0
+    refused = normal.copy()
+    refused[0, 1] = 2.0 ** -100
+    refused[M - 1, 3] = 3e38
+    s = gs.Sampler(vocab_size=V, max_rows=1)
+    try:
+        sc = torch.from_numpy(scales).cuda()
+        row = torch.from_numpy(words.view(np.int32)).cuda()
+        block = torch.from_numpy(oracle.repack_block_major(words, V, D).view(np.int32)).cuda()
+        for name, x in (("normal", normal), ("wide", wide), ("integers", integers), ("mixed", mixed),
+                        ("refused", refused)):
+            x = x.astype(np.float32)
+            want = np.stack([oracle.qat_linear_int2(x[m], words, scales, D, V, in_scale, 0.0) for m in range(M)])
+            xs = torch.from_numpy(x).cuda()
+            for layout, codes in ((gs.runtime.GS_QAT_ROW_MAJOR, row), (gs.runtime.GS_QAT_BLOCK_MAJOR, block)):
+                got = s.qat_lmhead(xs, codes, sc, layout=layout, input_scale=in_scale).cpu().numpy()
+                bad = np.nonzero(got.view(np.uint32) != want.view(np.uint32))
+                assert bad[0].size == 0, (name, layout, bad[0][:5], bad[1][:5], got[bad][:5], want[bad][:5])
+    finally:
+        s.close()
