@@ -67,6 +67,21 @@ __device__ __forceinline__ double srq(double v, double s) {
   return (double)(float)(q * s);
 }
 
+// srq with r = 1 / s rounded to nearest (0 where s lies outside 2^+-100: the
+// division): v / s in three operations, exactly rounded (Markstein; |v| is 0
+// or within 2^-300 .. 2^320 here, so nothing under- or overflows).
+__device__ __forceinline__ double srq_reciprocal(double s) { return s >= 0x1p-100 && s <= 0x1p100 ? 1.0 / s : 0.0; }
+__device__ __forceinline__ double srq(double v, double s, double r) {
+  if (r == 0) return srq(v, s);
+  const double q0 = v * r;
+  double ratio = __builtin_fma(__builtin_fma(-q0, s, v), r, q0);
+  ratio = v == 0 || v - v != 0 ? v : ratio;  // a zero keeps its sign; infinities and NaN
+  double q = __builtin_rint(ratio);
+  if (q == 0.0) q = ratio == 0.0 ? ratio : 0.0;
+  q = q < -128.0 ? -128.0 : (q > 127.0 ? 127.0 : q);
+  return (double)(float)(q * s);
+}
+
 // The activations of kRows rows of x from m0 (those below M) into act,
 // after the input SRQ, in binary64 (the whole block calls it).
 template <int kRows, int kThreads = kQatThreads>
@@ -374,14 +389,18 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
 //
 // Rows of x in groups of 16, a group's limbs resident in LDS for the whole
 // width: operand tile t holds the group's rows (kRows 16: limb t of each) or
-// limbs 2t and 2t + 1 of eight of them (kRows 8, where 16 rows' limbs would
-// not fit: more than 144 KB). A workgroup takes a run of 32-row vocabulary
+// limbs 2t and 2t + 1 of eight of them (kRows 8, where 16 rows' limbs take
+// more than 144 KB). A workgroup takes a run of 32-row vocabulary
 // pairs, a pair per wave: each code word is expanded once and multiplied by
 // every tile, and each limb tile read from LDS serves two vocabulary tiles
 // (64 lanes x 16 bytes per 32 cycles of a CU's matrix cores). Only as many
 // limbs are multiplied as the group's largest |A_k| has: 5 for activations of
 // an input SRQ, 5 or 6 for normal ones. The groups of one run are on one XCD,
-// so its codes come from HBM once.
+// so its codes come from HBM once. V 262144, D 1536, input SRQ: 3 rows
+// 40 us, 16 rows 59, 32 rows 81, 48 rows 106 (714 by qat_tile_kernel, a launch
+// per two rows), 64 rows 129; D 2048 without SRQ, 48 rows (eight at a time)
+// 194. Bound by the limbs read from LDS and the matrix cores (38 us each at
+// 48 rows); the check and the limbs take about 10 us a workgroup.
 constexpr int kQatGemmThreads = 512;
 constexpr int kQatGemmWaves = kQatGemmThreads / 64;
 constexpr int kQatGroup = 16;
@@ -402,60 +421,55 @@ union __attribute__((aligned(16))) QatGemmOp {
   double act[2 * 2048];        // the binary64 path's activations
 };
 
-// The first `limbs` limbs of 16 activations, word W of row o of the group (row
-// o of eight for kRows 8), at their operand positions (see above).
+// Bytes i of the four words into dword i (byte k of it from word k).
+__device__ __forceinline__ void transpose_bytes(const uint32_t (&w)[4], uint32_t (&d)[4]) {
+  const uint32_t a = __builtin_amdgcn_perm(w[1], w[0], 0x05010400u), b = __builtin_amdgcn_perm(w[1], w[0], 0x07030602u);
+  const uint32_t c = __builtin_amdgcn_perm(w[3], w[2], 0x05010400u), e = __builtin_amdgcn_perm(w[3], w[2], 0x07030602u);
+  d[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+  d[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+  d[2] = __builtin_amdgcn_perm(e, b, 0x05040100u);
+  d[3] = __builtin_amdgcn_perm(e, b, 0x07060302u);
+}
+
+// The first `limbs` limbs of 16 integers (below 2^52), word W of row o of the
+// group (row o of eight for kRows 8), at their operand positions (see above).
 template <int kRows>
-__device__ __forceinline__ void qat_store_limbs(i32x4* op, int steps, int limbs, int o, int W, const int64_t (&A)[16]) {
+__device__ __forceinline__ void qat_store_limbs(i32x4* op, int steps, int limbs, int o, int W, const double (&A)[16]) {
   constexpr uint64_t kK = 0x0080808080808080ull;
   const int step = 4 * (W >> 4) + (W & 3), gw = (W >> 2) & 3;
+  uint32_t dw[8][4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    uint32_t lo[4], hi[4];
+    uint32_t lo[4], hi[4], d[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint64_t u = ((uint64_t)A[4 * i + t] + kK) ^ kK;
+      // the integer's two halves: whole numbers, each step exact
+      const double h = __builtin_floor(A[4 * i + t] * 0x1p-32);
+      const uint64_t v = ((uint64_t)(uint32_t)(int)h << 32) | (uint32_t)__builtin_fma(h, -0x1p32, A[4 * i + t]);
+      const uint64_t u = (v + kK) ^ kK;
       lo[i] = (uint32_t)u;
       hi[i] = (uint32_t)(u >> 32);
     }
+    transpose_bytes(lo, d);
 #pragma unroll
-    for (int l = 0; l < 8; ++l) {
-      if (l >= limbs) break;
-      uint32_t dw = 0u;
+    for (int l = 0; l < 4; ++l) dw[l][t] = d[l];
+    transpose_bytes(hi, d);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dw |= (((l < 4 ? lo[i] : hi[i]) >> (8 * (l & 3))) & 0xFFu) << (8 * i);
-      const int tile = kRows == 16 ? l : l >> 1, at = kRows == 16 ? o : 8 * (l & 1) + o;
-      ((uint32_t*)&op[(tile * steps + step) * 64 + at + 16 * gw])[t] = dw;
-    }
+    for (int l = 0; l < 4; ++l) dw[4 + l][t] = d[l];
   }
-}
-
-// Integers A_k = a_k / 2^E of 16 activations; false past the bound.
-__device__ __forceinline__ bool qat_integers(const float (&f)[16], int E, int64_t (&A)[16], uint64_t* sabs,
-                                             uint64_t* ssum, uint64_t* largest) {
-  bool ok = true;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    A[e] = 0;
-    uint32_t sig = 0;
-    int g = 0;
-    if (!act_parts(f[e], &sig, &g) || !sig) continue;
-    const int sh = g - E;
-    if (sh > 62 - 24) { ok = false; continue; }
-    const uint64_t mag = (uint64_t)sig << sh;
-    if (mag >= kQatSumBound) { ok = false; continue; }
-    A[e] = f[e] < 0.0f ? -(int64_t)mag : (int64_t)mag;
-    *sabs += mag;
-    *ssum += (uint64_t)A[e];
-    *largest = mag > *largest ? mag : *largest;
+  for (int l = 0; l < 8; ++l) {
+    if (l >= limbs) break;
+    const int tile = kRows == 16 ? l : l >> 1, at = kRows == 16 ? o : 8 * (l & 1) + o;
+    op[(tile * steps + step) * 64 + at + 16 * gw] = i32x4{(int)dw[l][0], (int)dw[l][1], (int)dw[l][2], (int)dw[l][3]};
   }
-  return ok;
 }
 
 // The run's vocabulary pairs [p_lo, p_hi) against rows r0 .. r0 + kRows - 1 of
 // the group at m0, its limbs in op.
 template <int kTiles, int kRows>
 __device__ __forceinline__ void qat_gemm_run(const QatArgs& a, const QatGroupRows& R, const i32x4* op, int m0, int r0,
-                                             int rows_here, uint32_t ok_rows, int p_lo, int p_hi, bool cached) {
+                                             int rows_here, uint32_t ok_rows, int p_lo, int p_hi) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
   const int D = a.D, words = D / 16, blocks = D / 64, quads = (D + 255) / 256, steps = 4 * quads;
   const __amdgpu_buffer_rsrc_t cr =
@@ -463,6 +477,7 @@ __device__ __forceinline__ void qat_gemm_run(const QatArgs& a, const QatGroupRow
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, (short)0, a.V * 4, kBufferWord3);
   const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.out + (int64_t)m0 * a.V), (short)0,
                                                                        rows_here * a.V * 4, kBufferWord3);
+  const double r_out = srq_reciprocal(a.out_scale);
   constexpr int kQuads = kQatMaxSteps / 4;
   u32x4 cw[2][kQuads];
   // block 4 q + g of vocabulary row n; rows past V, blocks past the width and
@@ -472,8 +487,7 @@ __device__ __forceinline__ void qat_gemm_run(const QatArgs& a, const QatGroupRow
     const bool live = p < p_hi && n < (uint32_t)a.V && 4 * q + g < blocks;
     const uint32_t off = a.block_major ? ((uint32_t)(4 * q + g) * (uint32_t)a.V + n) * 16u
                                        : (n * (uint32_t)words + (uint32_t)(16 * q + 4 * g)) * 4u;
-    cw[v][q] = cached ? __builtin_amdgcn_raw_buffer_load_b128(cr, live ? off : kBufferOutOfRange, 0, 0)
-                      : __builtin_amdgcn_raw_buffer_load_b128(cr, live ? off : kBufferOutOfRange, 0, kQatNT);
+    cw[v][q] = __builtin_amdgcn_raw_buffer_load_b128(cr, live ? off : kBufferOutOfRange, 0, 0);
   };
   // no branch around a load (see above): quads past the width read zeros
   int p = p_lo + wave;
@@ -540,7 +554,7 @@ __device__ __forceinline__ void qat_gemm_run(const QatArgs& a, const QatGroupRow
         const int r = r0 + (kRows == 16 ? 4 * g + e : 4 * (g & 1) + e);
         const int64_t T = (int64_t)(s - 2 * (uint64_t)R.ssum[r]);
         const double dot = __builtin_ldexp((double)T, R.emin[r] != 0x7FFFFFFF ? R.emin[r] : 0);
-        const float y = (float)srq(dot * (double)sc[v], a.out_scale);
+        const float y = (float)srq(dot * (double)sc[v], a.out_scale, r_out);
         const uint32_t n = n0 + 16u * v;
         const bool st = (ok_rows >> r & 1u) != 0 && n < (uint32_t)a.V && (kRows == 16 || g < 2);
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), orr,
@@ -560,106 +574,127 @@ __global__ __launch_bounds__(kQatGemmThreads) void qat_gemm_kernel(QatArgs a, in
   const int group = in_band / 8, run = 8 * band + in_band % 8;
   if (run >= n_runs) return;
   const int m0 = kQatGroup * group;
+  const double r_in = srq_reciprocal(a.in_scale);
   const int rows_here = a.M - m0 < kQatGroup ? a.M - m0 : kQatGroup;
   const int n_pairs = (a.V + 31) / 32;
   const int p_lo = (int)((int64_t)run * n_pairs / n_runs), p_hi = (int)((int64_t)(run + 1) * n_pairs / n_runs);
   if (tid < kQatGroup) { R.emin[tid] = 0x7FFFFFFF; R.bad[tid] = 0; R.sabs[tid] = 0; R.ssum[tid] = 0; }
   if (tid == 0) R.limbs = 0;
   __syncthreads();
-  // the group's activations, after the input SRQ, by words of 16: thread t
-  // takes words t, t + kQatGemmThreads, ..
+  // The check: a row's activations after the input SRQ into LDS with their
+  // smallest granule, then the integers' sums. A row is one wave's, or
+  // several waves' when the rows are few; values are reduced in the wave (LDS
+  // atomics of every lane on one address took 20 us for 16 rows).
   const float4* x = (const float4*)(a.x + (int64_t)m0 * D);
-  const int n_words = rows_here * words;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int per_row = rows_here > 4 ? 1 : (rows_here > 2 ? 2 : (rows_here > 1 ? 4 : 8));
+  const int part = wave % per_row, row_step = kQatGemmWaves / per_row;
 #pragma unroll 1
-  for (int k = tid; k < n_words; k += kQatGemmThreads) {
+  for (int o = wave / per_row; o < rows_here; o += row_step) {
     int gmin = 0x7FFFFFFF;
     bool bad = false;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      float4 q = x[4 * k + v];
-      float e[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        e[i] = (float)srq((double)e[i], a.in_scale);
-        uint32_t sig;
-        int g;
-        if (!act_parts(e[i], &sig, &g)) bad = true;
-        else if (sig) gmin = g < gmin ? g : gmin;
-      }
-      L.f[4 * k + v] = make_float4(e[0], e[1], e[2], e[3]);
-    }
-    if (gmin != 0x7FFFFFFF) atomicMin(&R.emin[k / words], gmin);
-    if (bad) atomicOr(&R.bad[k / words], 1u);
-  }
-  auto activations = [&](int k, float (&f)[16]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float4 q = L.f[4 * k + v];
-      f[4 * v] = q.x; f[4 * v + 1] = q.y; f[4 * v + 2] = q.z; f[4 * v + 3] = q.w;
-    }
-  };
-  __syncthreads();
-  uint64_t largest = 0;
 #pragma unroll 1
-  for (int k = tid; k < n_words; k += kQatGemmThreads) {
-    const int o = k / words;
-    float f[16];
-    activations(k, f);
-    int64_t A[16];
-    uint64_t sabs = 0, ssum = 0, big = 0;
-    const bool ok = qat_integers(f, R.emin[o] != 0x7FFFFFFF ? R.emin[o] : 0, A, &sabs, &ssum, &big);
-    atomicAdd(&R.sabs[o], (unsigned long long)sabs);
-    atomicAdd(&R.ssum[o], (unsigned long long)ssum);
-    if (!ok) atomicOr(&R.bad[o], 1u);
-    largest = big > largest ? big : largest;
-  }
-  {
-    // n limbs hold |A| up to 0x7F7F .. 7F (n bytes)
-    uint32_t limbs = 1;
+    for (int W = 64 * part + lane; W < words; W += 64 * per_row) {
+      const int k = o * words + W;
 #pragma unroll
-    for (int n = 1; n < kQatLimbs; ++n) limbs += largest > (0x007F7F7F7F7F7F7Full >> (8 * (kQatLimbs - n))) ? 1u : 0u;
-    limbs = wave_max_u32(limbs);
-    if ((tid & 63) == 0) atomicMax(&R.limbs, limbs);
+      for (int v = 0; v < 4; ++v) {
+        const float4 q = x[4 * k + v];
+        float e[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          e[i] = (float)srq((double)e[i], a.in_scale, r_in);
+          uint32_t sig;
+          int g;
+          if (!act_parts(e[i], &sig, &g)) bad = true;
+          else if (sig) gmin = g < gmin ? g : gmin;
+        }
+        L.f[4 * k + v] = make_float4(e[0], e[1], e[2], e[3]);
+      }
+    }
+    // (granules are above -256: offset, they are unsigned, below "none")
+    const uint32_t least = wave_min_u32(gmin == 0x7FFFFFFF ? 0x7FFFFFFFu : (uint32_t)(gmin + 256));
+    const bool any_bad = __ballot(bad) != 0;
+    if (lane == 0) {
+      if (least != 0x7FFFFFFFu) atomicMin(&R.emin[o], (int)least - 256);
+      if (any_bad) atomicOr(&R.bad[o], 1u);
+    }
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int o = wave / per_row; o < rows_here; o += row_step) {
+    // The integers A_k = a_k / 2^E and their sums in binary64: whole numbers,
+    // exact below 2^53, and a sum that leaves that range stays out of it (an
+    // infinity or a NaN among them too).
+    double sabs = 0.0, ssum = 0.0, largest = 0.0;
+    const int E = R.emin[o] != 0x7FFFFFFF ? R.emin[o] : 0;
+#pragma unroll 1
+    for (int W = 64 * part + lane; W < words; W += 64 * per_row) {
+      const int k = o * words + W;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float4 q = L.f[4 * k + v];
+        const float e[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double A = __builtin_ldexp((double)e[i], -E);
+          sabs += fabs(A);
+          ssum += A;
+          largest = fmax(largest, fabs(A));
+        }
+      }
+    }
+    sabs = wave_sum_f64_dpp(sabs);
+    ssum = wave_sum_f64_dpp(ssum);
+    const bool fits = sabs < (double)kQatSumBound;
+    const uint64_t most = wave_max_u64(fits ? (uint64_t)largest : 0ull);
+    if (lane == 0) {
+      // n limbs hold |A| up to 0x7F7F .. 7F (n bytes)
+      uint32_t limbs = 1;
+      for (int n = 1; n < kQatLimbs; ++n) limbs += most > (0x007F7F7F7F7F7F7Full >> (8 * (kQatLimbs - n))) ? 1u : 0u;
+      atomicAdd(&R.sabs[o], (unsigned long long)(fits ? sabs : 0.0));
+      atomicAdd(&R.ssum[o], (unsigned long long)(int64_t)(fits ? ssum : 0.0));
+      if (!fits) atomicOr(&R.bad[o], 1u);
+      atomicMax(&R.limbs, limbs);
+    }
   }
   __syncthreads();
   uint32_t ok_rows = 0;
   for (int o = 0; o < rows_here; ++o) ok_rows |= !R.bad[o] && R.sabs[o] < kQatSumBound ? 1u << o : 0u;
   const int limbs = (int)R.limbs < kQatMinTiles ? kQatMinTiles : (int)R.limbs;
-  const bool cached = n_groups > 1;
 
   // The limbs take the activations' place in LDS, so these are read again.
-  // (Limbs of a refused row reach only outputs that are not stored.)
-  auto word = [&](int k, int64_t (&A)[16]) __attribute__((always_inline)) {
-    float e[16];
+  // A refused row's limbs are zeros.
+  auto word = [&](int o, int W, double (&A)[16]) __attribute__((always_inline)) {
+    const int E = R.emin[o] != 0x7FFFFFFF ? R.emin[o] : 0;
+    const bool ok = (ok_rows >> o & 1u) != 0;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const float4 q = x[4 * k + v];
-      e[4 * v] = (float)srq((double)q.x, a.in_scale);
-      e[4 * v + 1] = (float)srq((double)q.y, a.in_scale);
-      e[4 * v + 2] = (float)srq((double)q.z, a.in_scale);
-      e[4 * v + 3] = (float)srq((double)q.w, a.in_scale);
+      const float4 q = x[4 * (o * words + W) + v];
+      const float e[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        A[4 * v + i] = ok ? __builtin_ldexp((double)(float)srq((double)e[i], a.in_scale, r_in), -E) : 0.0;
     }
-    uint64_t u0 = 0, u1 = 0, u2 = 0;
-    const int E = R.emin[k / words];
-    (void)qat_integers(e, E != 0x7FFFFFFF ? E : 0, A, &u0, &u1, &u2);
   };
   if (ok_rows == 0) {
     // nothing for the integer path
   } else if (limbs * steps * 1024 <= kQatOpBytes) {
     __syncthreads();
 #pragma unroll 1
-    for (int k = tid; k < n_words; k += kQatGemmThreads) {
-      int64_t A[16];
-      word(k, A);
-      qat_store_limbs<16>(L.op, steps, limbs, k / words, k % words, A);
+    // (lanes along the rows: their 16-byte pieces are neighbours in LDS)
+    for (int k = tid; k < rows_here * words; k += kQatGemmThreads) {
+      const int o = k % rows_here, W = k / rows_here;
+      double A[16];
+      word(o, W, A);
+      qat_store_limbs<16>(L.op, steps, limbs, o, W, A);
     }
     __syncthreads();
     switch (limbs) {
-      case 3: qat_gemm_run<3, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
-      case 4: qat_gemm_run<4, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
-      case 5: qat_gemm_run<5, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
-      case 6: qat_gemm_run<6, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
-      default: qat_gemm_run<7, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi, cached); break;
+      case 3: qat_gemm_run<3, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi); break;
+      case 4: qat_gemm_run<4, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi); break;
+      case 5: qat_gemm_run<5, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi); break;
+      case 6: qat_gemm_run<6, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi); break;
+      default: qat_gemm_run<7, 16>(a, R, L.op, m0, 0, rows_here, ok_rows, p_lo, p_hi); break;
     }
   } else {
     // eight rows at a time, all limbs (4 tiles: 128 KB at width 2048)
@@ -667,15 +702,16 @@ __global__ __launch_bounds__(kQatGemmThreads) void qat_gemm_kernel(QatArgs a, in
     for (int r0 = 0; r0 < rows_here; r0 += 8) {
       __syncthreads();
 #pragma unroll 1
-      for (int k = tid; k < n_words; k += kQatGemmThreads) {
-        const int o = k / words;
-        if (o < r0 || o >= r0 + 8) continue;
-        int64_t A[16];
-        word(k, A);
-        qat_store_limbs<8>(L.op, steps, 8, o - r0, k % words, A);
+      for (int k = tid; k < 8 * words; k += kQatGemmThreads) {
+        const int o = k & 7, W = k / 8;
+        if (r0 + o >= rows_here) continue;
+        double A[16];
+        word(r0 + o, W, A);
+        qat_store_limbs<8>(L.op, steps, 8, o, W, A);
       }
       __syncthreads();
-      qat_gemm_run<4, 8>(a, R, L.op, m0, r0, rows_here, ok_rows, p_lo, p_hi, cached);
+      if (limbs <= 6) qat_gemm_run<3, 8>(a, R, L.op, m0, r0, rows_here, ok_rows, p_lo, p_hi);
+      else qat_gemm_run<4, 8>(a, R, L.op, m0, r0, rows_here, ok_rows, p_lo, p_hi);
     }
   }
   // rows the check refused: the binary64 path over this run's vocabulary rows
@@ -706,16 +742,20 @@ void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* wor
   QatArgs a{x, words, scales, out, D, V, M, block_major, in_scale, out_scale};
   const int cus = cu_count > 0 ? cu_count : 256;
   if (D % 256 == 0 && D <= 2048 && V % 16 == 0 && M <= 2) {
-    // one or two rows: one workgroup per compute unit
+    // one or two rows: one workgroup per compute unit, the codes streamed past
+    // eight limb rows (24 us at V 262144, D 1536; qat_gemm_kernel 36)
     hipExtLaunchKernelGGL(qat_tile_kernel, dim3(cus), dim3(kQatTileThreads), 0, s, ev.start, ev.stop, 0, a, 0);
     return;
   }
   if (D <= 2048) {
-    // groups of 16 rows, about one workgroup per compute unit in all
+    // groups of 16 rows, about one workgroup per compute unit in all (3 rows of
+    // V 262144, D 1536 take 40 us, two launches of the kernel above 48)
     const int groups = (M + kQatGroup - 1) / kQatGroup;
     const int pairs = (V + 31) / 32;
-    int runs = cus / groups;
-    runs = runs < 1 ? 1 : (runs > pairs ? pairs : runs);
+    // as many runs as each XCD's compute units take at once: one workgroup
+    // more on some of them doubled the time (48 rows in 85 runs 235 us)
+    int runs = 8 * (cus / 8 / groups);
+    runs = runs < 8 ? 8 : (runs > pairs ? pairs : runs);
     hipExtLaunchKernelGGL(qat_gemm_kernel, dim3(((runs + 7) / 8) * 8 * groups), dim3(kQatGemmThreads), 0, s, ev.start,
                           ev.stop, 0, a, groups, runs);
     return;
