@@ -2272,7 +2272,7 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
   // (with a full pool: u * 1, the prefix sums carrying the normaliser's error,
   // settled again with the recomputed normaliser when within that margin)
   const double u = u_draw;
-  {
+  for (;;) {
     double local[kPer];
     double s = 0.0;
     for (int q = 0; q < kPer; ++q) {
@@ -2320,6 +2320,19 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
         S.deep_margin = full_mass_rel + kNearTie;
       }
       return kDeepRequest;
+    }
+    if (full_mass && pre_cut && !refined && S.route_exact == 8u && !S.short_sum) {
+      // a full-vocabulary draw within the scan normaliser's margin among the
+      // candidates ranked up to its cursor: the normaliser recomputed, and
+      // the draw again (two rows in a thousand of N(0, 9) logits; their
+      // replays, 17.6 ms each, were most of a batch's time)
+      __syncthreads();
+      if (tid == 0) { S.route_exact = 0; S.first_idx = 0xFFFFFFFFu; }
+      if (!refine()) {
+        return kExactRequest | GS_FLAG_NEAR_TIE;
+      }
+      __syncthreads();
+      continue;
     }
     if (S.route_exact || S.first_idx == 0xFFFFFFFFu || S.short_sum) {
       // a near tie, or a full-vocabulary draw past the ranked candidates

@@ -354,3 +354,39 @@ def test_typical_p_ties_and_small_pools(oracle):
     finally:
         s.close()
     check(gs, oracle, "typical small", out, rows, None, cfgs, us)
+
+
+@pytest.mark.parametrize("n_hist", [0, 30])
+def test_full_vocabulary_draw_within_the_scan_margin(sampler, oracle, n_hist):
+    """u within the scan normaliser's margin (3.9e-7) of a prefix sum past the
+    top 64: the normaliser is recomputed in binary64 and settles the draw
+    (its margin is 4e-9), with and without special ids; within 1e-11 the row
+    is replayed. Ids are the oracle's either way."""
+    import torch
+
+    gs = _gs()
+    rng = np.random.default_rng(29)
+    x = rng.normal(0, 3, V).astype(np.float32)
+    T = 0.8
+    hist = np.argsort(-x)[:n_hist].tolist()
+    v = x.astype(np.float64)
+    for i in hist:
+        v[i] = v[i] / 1.2
+    v = np.sort(v / T)[::-1]
+    e = np.exp(v - v[0])
+    cum = np.cumsum(e / e.sum())
+    us, near = [], []
+    for i in (100, 300, 700, 1500):
+        for d in (-1e-7, 1e-7, -2e-8, 2e-8, 1e-11):
+            us.append(float(cum[i] + d))
+            near.append(abs(d) < 1e-10)
+    cfg = gs.DecodingConfig(temperature=T, topK=0, topP=1.0, repetitionPenalty=1.2 if n_hist else 1.0,
+                            repetitionWindow=64 if n_hist else 0)
+    cfgs, hists = [cfg] * len(us), [hist] * len(us)
+    conf = np.stack([gs.runtime.row_config(c, uniform=u) for c, u in zip(cfgs, us)])
+    dev = torch.from_numpy(np.stack([x] * len(us))).cuda()
+    for hints in (None, 0):
+        out = sampler.sample(dev, conf, histories=hists, hints=hints)
+        check(gs, oracle, "scan margin", out, [x] * len(us), hists, cfgs, us)
+        exact = (out.flags & gs.GS_FLAG_EXACT_PATH) != 0
+        assert np.array_equal(exact, np.array(near)), (hints, list(zip(us, exact)))
