@@ -2046,6 +2046,7 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
   // them all. The top-p pass checks the mass it sums over them.
   int n_pre = n_ns, n_sp_pre = n_sp_in;
   bool pre_cut = false;  // the ranked candidates end before the region does
+  uint32_t pre_floor = 0;  // the logit key they end at
   // a draw whose pool is the whole row (the draw's margin as below)
   const bool draw_pool = cfg.top_p >= 1 && cfg.top_k <= 0 && !(cfg.min_p > 0) && !constrained;
   const double u_draw = cfg.rng_mode == GS_RNG_EXPLICIT ? cfg.uniform : gsm::mulberry32_draw(cfg.seed, cfg.draw_index);
@@ -2112,6 +2113,7 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
       }
       n_sp_pre = lo;
       pre_cut = true;
+      pre_floor = floor_key;
     }
     const uint64_t* src = pre_cut ? scratch : S.sorted;
     const int len = pow2_at_least(n_pre);
@@ -2272,7 +2274,7 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
   // (with a full pool: u * 1, the prefix sums carrying the normaliser's error,
   // settled again with the recomputed normaliser when within that margin)
   const double u = u_draw;
-  for (;;) {
+  {
     double local[kPer];
     double s = 0.0;
     for (int q = 0; q < kPer; ++q) {
@@ -2308,31 +2310,21 @@ __device__ __forceinline__ uint32_t finish_row(const SampleArgs& a, FinishLds& U
       if (wave_near) atomicOr(&S.route_exact, 8u);
     }
     __syncthreads();
-    if (full_mass && !constrained && !pre_cut && (S.route_exact == 8u || S.first_idx == 0xFFFFFFFFu)) {
+    if (full_mass && !constrained && (S.route_exact == 8u || S.first_idx == 0xFFFFFFFFu || S.short_sum)) {
       // a full-vocabulary draw within the scan normaliser's margin or past
-      // the region: the deep draw takes it from the region's candidates
+      // the ranked candidates: the deep draw takes it from these, every
+      // candidate down to the region's floor or to the one the ranking
+      // stopped at (such rows, two in a thousand of N(0, 9) logits, were
+      // replayed: 17.6 ms, most of a batch's time)
       if (tid == 0) {
         S.deep_m = M;
         S.deep_u = u;
-        S.deep_thr = thr;
-        S.deep_floor = region_floor;
+        S.deep_thr = pre_cut ? pre_floor : thr;
+        S.deep_floor = pre_cut ? f64_key((double)key_f32(pre_floor) / T) : region_floor;
         S.deep_n = (uint32_t)n;
         S.deep_margin = full_mass_rel + kNearTie;
       }
       return kDeepRequest;
-    }
-    if (full_mass && pre_cut && !refined && S.route_exact == 8u && !S.short_sum) {
-      // a full-vocabulary draw within the scan normaliser's margin among the
-      // candidates ranked up to its cursor: the normaliser recomputed, and
-      // the draw again (two rows in a thousand of N(0, 9) logits; their
-      // replays, 17.6 ms each, were most of a batch's time)
-      __syncthreads();
-      if (tid == 0) { S.route_exact = 0; S.first_idx = 0xFFFFFFFFu; }
-      if (!refine()) {
-        return kExactRequest | GS_FLAG_NEAR_TIE;
-      }
-      __syncthreads();
-      continue;
     }
     if (S.route_exact || S.first_idx == 0xFFFFFFFFu || S.short_sum) {
       // a near tie, or a full-vocabulary draw past the ranked candidates

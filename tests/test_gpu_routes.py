@@ -359,9 +359,9 @@ def test_typical_p_ties_and_small_pools(oracle):
 @pytest.mark.parametrize("n_hist", [0, 30])
 def test_full_vocabulary_draw_within_the_scan_margin(sampler, oracle, n_hist):
     """u within the scan normaliser's margin (3.9e-7) of a prefix sum past the
-    top 64: the normaliser is recomputed in binary64 and settles the draw
-    (its margin is 4e-9), with and without special ids; within 1e-11 the row
-    is replayed. Ids are the oracle's either way."""
+    top 64: the deep draw settles it from the candidates ranked up to the
+    cursor (its margin is 1.6e-10), with and without special ids; within
+    1e-11 the row is replayed. Ids are the oracle's either way."""
     import torch
 
     gs = _gs()
