@@ -14,7 +14,9 @@
 // sums move by V 2^-53 relative) is left to the exact replay: a sum within
 // `margin` of its threshold, two different logits whose surprises differ by
 // less than the entropy's error at the cut, two whose probabilities could
-// round either way at the draw.
+// round either way at the draw. The bins' sums vary in their last bits with
+// the order of the LDS atomics: no decision rests on those, only, within
+// 1e-15 of the margin's own edge, whether the replay takes it.
 //
 // Bound by the exponential pass on one CU (about 30 binary64 operations a
 // logit); more workgroups a row would need a launch for each of the four
