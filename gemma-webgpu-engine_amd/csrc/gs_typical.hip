@@ -263,7 +263,8 @@ __device__ __forceinline__ bool typ_settle(const SampleArgs& a, TypicalLds& S, i
     const double x = below(l);
     const int b = live ? bin(x) : -1;
     const bool pass = b >= o0 && b < o1 && !(b >= i0 && b < i1);
-    typ_append(S, pass, gsm::bits_of(fabs(x - c)), ((uint64_t)__builtin_bit_cast(uint32_t, l) << 32) | id);
+    // (the key joins the zeros: equal values are in order of id alone)
+    typ_append(S, pass, gsm::bits_of(fabs(x - c)), ((uint64_t)f32_key(l) << 32) | id);
   });
   __syncthreads();
   int n = (int)S.n;
@@ -273,7 +274,7 @@ __device__ __forceinline__ bool typ_settle(const SampleArgs& a, TypicalLds& S, i
   constexpr int kOwn = kTypCap / kTypThreads;
   const double margin = z * fmax(kNearTie, 4.0 * V * 0x1p-53);
   auto logit_of = [&](uint64_t k2) __attribute__((always_inline)) -> float {
-    return __builtin_bit_cast(float, (uint32_t)(k2 >> 32));
+    return key_f32((uint32_t)(k2 >> 32));
   };
   // the first entry whose running sum from `from` reaches `want`, -1 when a
   // sum lies within the margin of it; in every thread, with the sum there

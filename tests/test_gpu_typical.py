@@ -67,3 +67,72 @@ def test_typical_rows_match_the_oracle(oracle, V, pad, dtype):
             assert names[r] != "equal" and (names[r] != "masked" or caps[r] > 0), (names[r], r)
             assert abs(out.probabilities[r] - tr.probability) <= V * 2.0 ** -52 * tr.probability, (names[r], r)
     assert settled >= len(cfgs) // 3, settled
+
+
+def _softmax(x, T):
+    """Probabilities and surprises of a row in binary64 (the typical order's inputs)."""
+    v = x.astype(np.float64) / T
+    p = np.exp(v - v.max())
+    p /= p.sum()
+    return p, np.abs(-np.log(p) + np.sum(p * np.log(p)))
+
+
+def _cuts_within(x, T, group, fractions, picks):
+    """(typicalP, u) with the typical cut inside the items `group` (a boolean mask of equal surprise), at the
+    fractions of their mass (never at an item's end), and draws at the picks of the kept part of it."""
+    p, s = _softmax(x, T)
+    edge = s[group].max() + 1e-9
+    nearer = (s < edge) & ~group
+    before, mass = p[nearer].sum(), p[group].sum()
+    above = p[nearer & (p > p[group].max())].sum()
+    n = int(group.sum())
+    for f in fractions:
+        f = (np.floor(f * n) + 0.4) / n
+        kept = before + f * mass
+        for g in picks:
+            yield kept, (above + g * f * mass) / kept
+
+
+def _check_rows(oracle, rows, dtype):
+    """Samples rows [(name, x, T, typicalP, u)]; ids must be the oracle's. Returns which were replayed."""
+    import torch
+
+    import gsample as gs
+
+    V = len(rows[0][1])
+    x = torch.from_numpy(np.stack([r[1] for r in rows]).astype(np.float32)).to(dtype)
+    cfgs = [gs.DecodingConfig(temperature=r[2], topK=0, topP=1.0, typicalP=r[3], repetitionPenalty=1.0,
+                              repetitionWindow=0) for r in rows]
+    s = gs.Sampler(vocab_size=V, max_rows=len(rows))
+    try:
+        conf = np.stack([gs.runtime.row_config(c, uniform=r[4]) for c, r in zip(cfgs, rows)])
+        out = s.sample(x.cuda(), conf)
+    finally:
+        s.close()
+    values = x.to(torch.float32).numpy()
+    for i, (name, _, T, p, u) in enumerate(rows):
+        t, _ = oracle.sample_token(values[i], [], Decoding(temperature=T, topK=0, topP=1.0, minP=0.0, typicalP=p,
+                                                           repetitionPenalty=1.0, repetitionWindow=0), u)
+        assert int(out.tokens[i]) == t, (name, T, p, u, int(out.tokens[i]), t)
+    return (out.flags & gs.GS_FLAG_EXACT_PATH) != 0
+
+
+def _zeros_rows(rng, V=2048):
+    """Rows of a grid with zeros of both signs mixed, the cut and the draw among the zeros."""
+    for step in (0.25, 0.125, 0.5):
+        x = np.round(rng.normal(0, 3, V) / step) * step
+        x[rng.random(V) < 0.15] = 0.0
+        x = np.where((x == 0) & (rng.random(V) < 0.5), -0.0, x)
+        for T in (0.7, 1.3):
+            for p, u in _cuts_within(x, T, x == 0, (0.2, 0.5, 0.8), (0.1, 0.5, 0.9)):
+                yield f"zeros {step}", x, T, p, u
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_typical_cut_among_signed_zeros(oracle, dtype):
+    """+0 and -0 are equal: the zeros kept are the ones of the lowest ids, whatever their sign."""
+    import torch
+
+    rows = list(_zeros_rows(np.random.default_rng(5)))
+    replayed = _check_rows(oracle, rows, getattr(torch, dtype))
+    assert not replayed.any(), np.nonzero(replayed)[0]
