@@ -313,16 +313,29 @@ __device__ __forceinline__ bool typ_settle(const SampleArgs& a, TypicalLds& S, i
   double kept = 0.0;
   const int cut = reach(inner, target, false, &kept);
   if (cut < 0) return false;
+  // whether v holds in some thread (S.flag is 0: the reach before found its entry)
+  auto in_any = [&](bool v) __attribute__((always_inline)) -> bool {
+    if (__ballot(v) != 0 && lane == 0) atomicOr(&S.flag, 1u);
+    __syncthreads();
+    const bool r = S.flag != 0;
+    __syncthreads();
+    return r;
+  };
   {
-    // the reference's surprises differ from these by the entropy's error (the
-    // items before and after the list lie within lo, or past hi)
+    // the reference's surprises differ from these by the entropy's error: no
+    // other logit of the list within it (however many equal ones lie between),
+    // and none of the items before and after the list, which lie within lo or
+    // past hi
     const double err = 2.0 * (4.0 * V * 0x1p-53 * (gsm::js_log(z) + c + 2.0) + 1.0e-12);
     const double s = gsm::double_of(S.k1[cut]), slack = err + 1.0e-6 / per;
-    auto apart = [&](int i) __attribute__((always_inline)) -> bool {
-      return i < 0 || i >= n || logit_of(S.k2[i]) == logit_of(S.k2[cut]) || fabs(gsm::double_of(S.k1[i]) - s) >= err;
-    };
-    if (!apart(cut - 1) || !apart(cut + 1) || (w_lo >= 0 && s - w_lo / per < slack) || w_hi / per - s < slack)
-      return false;
+    const uint32_t key = (uint32_t)(S.k2[cut] >> 32);
+    bool near = false;
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+      const int i = tid * kOwn + k;
+      near |= i < n && (uint32_t)(S.k2[i] >> 32) != key && fabs(gsm::double_of(S.k1[i]) - s) < err;
+    }
+    if (in_any(near) || (w_lo >= 0 && s - w_lo / per < slack) || w_hi / per - s < slack) return false;
   }
 
   // ---- the draw (sampling.ts:58-64): by falling probability the kept items

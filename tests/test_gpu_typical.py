@@ -136,3 +136,43 @@ def test_typical_cut_among_signed_zeros(oracle, dtype):
     rows = list(_zeros_rows(np.random.default_rng(5)))
     replayed = _check_rows(oracle, rows, getattr(torch, dtype))
     assert not replayed.any(), np.nonzero(replayed)[0]
+
+
+def _mirrored_rows(rng, V=2048):
+    """Two groups of equal logits on either side of the mean, their surprises equal to rounding (the temperature
+    is found by bisection: 2 E[l] = 7 + 5), the cut among them."""
+    x = np.round(rng.normal(0, 3, V) * 8) / 8
+    x[(x == 7) | (x == 5)] = 0.125
+    ids = rng.permutation(V)
+    x[ids[:40]], x[ids[40:100]] = 7.0, 5.0
+    lo, hi = 0.3, 6.0  # E[l] falls as the temperature rises
+    for _ in range(200):
+        T = 0.5 * (lo + hi)
+        lo, hi = (T, hi) if float(np.sum(_softmax(x, T)[0] * x)) > 6.0 else (lo, T)
+    group = (x == 7) | (x == 5)
+    for T in (lo, hi, lo * (1 - 4e-16), hi * (1 + 4e-16), lo * (1 + 4e-15)):
+        for p, _ in _cuts_within(x, T, group, (0.2, 0.5, 0.8), (0.5,)):
+            for u in rng.random(6):
+                yield "mirrored", x, T, p, float(u)
+
+
+def _tiny_rows(rng, V=2048):
+    """Zeros with a few 3e-17 among them: other logits of the same surprise, the cut and the draw in the zeros."""
+    x = np.round(rng.normal(0, 3, V) * 4) / 4
+    x[rng.random(V) < 0.15] = 0.0
+    zeros = np.nonzero(x == 0)[0]
+    group = x == 0
+    x[zeros[[1, len(zeros) // 2, -1]]] = 3e-17
+    for T in (0.7, 1.3):
+        for p, u in _cuts_within(x, T, group, (0.2, 0.5, 0.8), (0.1, 0.5, 0.9)):
+            yield "tiny", x, T, p, u
+
+
+@pytest.mark.parametrize("make", [_mirrored_rows, _tiny_rows])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_typical_cut_between_equal_surprises(oracle, dtype, make):
+    """Different logits of one surprise at the cut: the reference's rounding orders them, however many
+    equal logits lie between the cut and the next different one, so the replay decides."""
+    import torch
+
+    assert _check_rows(oracle, list(make(np.random.default_rng(5))), getattr(torch, dtype)).all()
