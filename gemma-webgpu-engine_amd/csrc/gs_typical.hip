@@ -402,15 +402,24 @@ __device__ __forceinline__ bool typ_settle(const SampleArgs& a, TypicalLds& S, i
   const float l = key_f32(~(uint32_t)S.k1[hit]);
   const double x = below(l);
   {
-    // neighbours whose probabilities could round out of order: equal logits
-    // are in order of id, others lie apart, and a list's ends off the bin's
-    auto apart = [&](int i) __attribute__((always_inline)) -> bool {
-      return S.k1[i] == S.k1[hit] || fabs(below(key_f32(~(uint32_t)S.k1[i])) - x) > 1.0e-12;
-    };
-    const double f = x * per - __builtin_floor(x * per);
-    const bool wide = 1.0e-6 / per > 1.0e-12;
-    const bool before = hit > 0 ? apart(hit - 1) : x == 0.0 || (wide && f > 1.0e-6);
-    const bool after = hit + 1 < n ? apart(hit + 1) : wide && f < 1.0 - 1.0e-6;
+    // no other logit whose probability could round out of order: in the list
+    // (however many equal ones, in order of id, lie between), and, where the
+    // run of equal ones reaches the list's end, in the window's next bin past
+    // it. A bin there that moves no prefix sum is empty, or its items lie
+    // below the margin's resolution, where no draw settles.
+    const uint64_t key = S.k1[hit];
+    bool near = false;
+#pragma unroll
+    for (int k = 0; k < kOwn; ++k) {
+      const int i = tid * kOwn + k;
+      near |= i < n && S.k1[i] != key && fabs(below(key_f32(~(uint32_t)S.k1[i])) - x) <= 1.0e-12;
+    }
+    if (in_any(near)) return false;
+    const int b0 = in_bin >= 0 ? in_bin : (!upper ? i1 : 0);             // bins below b0 precede the list,
+    const int b1 = in_bin >= 0 ? in_bin + 1 : (!lower ? i0 : kTypBins);  // bins from b1 on follow it
+    const double edge = fmax(1.0e-6, 1.0e-12 * per);
+    const bool before = S.k1[0] != key || b0 == 0 || x * per - b0 > edge || S.mass[b0] == S.mass[b0 - 1];
+    const bool after = S.k1[n - 1] != key || b1 == kTypBins || b1 - x * per > edge || S.mass[b1 + 1] == S.mass[b1];
     if (!before || !after) return false;
   }
   if (tid == 0) {

@@ -176,3 +176,42 @@ def test_typical_cut_between_equal_surprises(oracle, dtype, make):
     import torch
 
     assert _check_rows(oracle, list(make(np.random.default_rng(5))), getattr(torch, dtype)).all()
+
+
+def _drawn(x, T):
+    """(typicalP, u) of draws in the middle of a row's zeros, the cut elsewhere."""
+    p, _ = _softmax(x, T)
+    zero = np.abs(x) < 1e-9
+    above, mass = p[x > 0.1].sum(), p[zero].sum()
+    return [(0.9999, (above + g * mass) / 0.9999) for g in (0.3, 0.5, 0.7)]
+
+
+def _tiny_drawn_rows(rng, V=2048):
+    """Zeros with a few 3e-17 among them, and zeros that start a bin (the row spans 64 grid steps, a power of
+    two) with a few 2e-15 at the end of the bin above."""
+    x = next(_tiny_rows(rng, V))[1]
+    for T in (1.3, 2.0):
+        for p, u in _drawn(x, T):
+            yield "tiny drawn", x, T, p, u
+    for _, x, T, p, u in list(_bin_edge_rows(rng, V)):
+        x = x.copy()
+        x[np.nonzero(x == 0)[0][[3, -2]]] = 2e-15
+        yield "tiny above the bin", x, T, p, u
+
+
+def _bin_edge_rows(rng, V=2048):
+    x = np.clip(np.round(rng.normal(0, 3, V) * 4) / 4, -8, 8)
+    x[[17, 1900]] = 8.0, -8.0
+    for p, u in _drawn(x, 1.0):
+        yield "bin edge", x, 1.0, p, u
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_typical_draw_between_equal_probabilities(oracle, dtype):
+    """Different logits whose probabilities could round out of order around the drawn one: the replay decides,
+    also with equal logits between them and the drawn one, or a bin's edge. A run of equal logits
+    at a bin's edge with nothing beyond it is settled."""
+    import torch
+
+    assert _check_rows(oracle, list(_tiny_drawn_rows(np.random.default_rng(5))), getattr(torch, dtype)).all()
+    assert not _check_rows(oracle, list(_bin_edge_rows(np.random.default_rng(5))), getattr(torch, dtype)).any()
