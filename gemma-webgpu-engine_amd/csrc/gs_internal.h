@@ -530,15 +530,16 @@ __device__ __forceinline__ void history_window(const SampleArgs& a, int64_t row,
   *end = h1;
 }
 
-// Rows of the typical-p kernel: typical-p alone over the whole vocabulary
-// (no penalties, mask, min-p, top-k or top-p), at temperatures where
-// div_by_temperature is the division.
+// Rows of the typical-p kernel, which the finish leaves to it: typical-p alone
+// over the whole vocabulary (no penalties, mask, min-p, top-k or top-p), at
+// temperatures where div_by_temperature is the division. With a topK of all
+// of at most kMaxFastK ids the finish settles the row itself.
 __device__ __forceinline__ bool typical_row(const SampleArgs& a, int64_t row, const gs_row_config& c) {
   int64_t w0, w1;
   history_window(a, row, c, &w0, &w1);
-  return c.typical_p > 0 && c.typical_p < 1 && (c.options & GS_ROW_FORCE_EXACT) == 0 &&
-         (c.top_k <= 0 || c.top_k >= a.vocab) && !(c.min_p > 0) && c.top_p >= 1 && c.mask_slot < 0 && w1 <= w0 &&
-         c.temperature >= 0x1p-20 && c.temperature <= 0x1p20;
+  return plan_row(c).route == kRouteExact && c.typical_p > 0 && c.typical_p < 1 &&
+         (c.options & GS_ROW_FORCE_EXACT) == 0 && (c.top_k <= 0 || c.top_k >= a.vocab) && !(c.min_p > 0) &&
+         c.top_p >= 1 && c.mask_slot < 0 && w1 <= w0 && c.temperature >= 0x1p-20 && c.temperature <= 0x1p20;
 }
 
 // -------------------------------------------- distinct ids of one row

@@ -3,6 +3,8 @@ probabilities equal on replayed rows, within V 2^-52 relative of the oracle's
 sequential sums on the rows that one pass settles. Sizes around the 16-byte
 pieces and the workgroup's stride, rows at every alignment, equal logits in
 one bin, heavy tails, softcap, and rows that only the replay settles."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -215,3 +217,51 @@ def test_typical_draw_between_equal_probabilities(oracle, dtype):
 
     assert _check_rows(oracle, list(_tiny_drawn_rows(np.random.default_rng(5))), getattr(torch, dtype)).all()
     assert not _check_rows(oracle, list(_bin_edge_rows(np.random.default_rng(5))), getattr(torch, dtype)).any()
+
+
+@pytest.mark.parametrize("V", [17, 40, 64, 65])
+def test_typical_rows_are_decided_once(oracle, V):
+    """A topK of the whole vocabulary: up to 64 the finish settles such rows (its flags and probabilities
+    stay, with the batch's typical-p hint too), past it the typical-p kernel. Through a context and
+    through the entry point with two replay slots."""
+    import torch
+
+    import gsample as gs
+
+    rng = np.random.default_rng(V)
+    rows, R = [], 48
+    for i in range(R):
+        x = np.full(V, 1.5) if i % 4 == 3 else rng.normal(0, 3, V)
+        rows.append(np.round(x * 4) / 4 if i % 2 else x)
+    x = torch.from_numpy(np.stack(rows).astype(np.float32)).cuda()
+    us = rng.random(R)
+    cfgs = [gs.DecodingConfig(temperature=0.8, topK=max(V, 64) if i % 3 == 0 else V, topP=1.0,
+                              typicalP=float(rng.uniform(0.2, 0.99)), repetitionPenalty=1.0, repetitionWindow=0)
+            for i in range(R)]
+    conf = np.stack([gs.runtime.row_config(c, uniform=u) for c, u in zip(cfgs, us)])
+    s = gs.Sampler(vocab_size=V, max_rows=R)
+    try:
+        plain = s.sample(x, conf, hints=0)
+        out = s.sample(x, conf)
+        assert s.prepare(x, conf)[0].hints & gs.runtime.GS_BATCH_TYPICAL
+        b, keep = s.prepare(x, conf)
+        res = torch.zeros((R, 2), dtype=torch.float64, device="cuda")
+        b.results = res.data_ptr()
+        torch.cuda.synchronize()
+        stream = torch.cuda.Stream()
+        assert gs.runtime.library().gs_sample_noalloc(C.byref(b), V, C.c_void_p(stream.cuda_stream)) == 0
+        stream.synchronize()
+        fixed = res.cpu().numpy().view(np.uint8).reshape(-1).view(gs.runtime.RESULT_DTYPE)
+    finally:
+        s.close()
+    for i, c in enumerate(cfgs):
+        t, _ = oracle.sample_token(x[i].cpu().numpy(), [], Decoding(
+            temperature=c.temperature, topK=c.topK, topP=1.0, minP=0.0, typicalP=c.typicalP, repetitionPenalty=1.0,
+            repetitionWindow=0), us[i])
+        assert int(plain.tokens[i]) == int(out.tokens[i]) == int(fixed["token"][i]) == t, i
+    assert np.array_equal(out.flags, fixed["flags"])
+    assert np.array_equal(out.probabilities, fixed["probability"])
+    if V <= 64:
+        assert np.array_equal(out.flags, plain.flags) and np.array_equal(out.probabilities, plain.probabilities)
+    else:
+        assert (plain.flags & gs.GS_FLAG_EXACT_PATH).all() and not (out.flags & gs.GS_FLAG_EXACT_PATH).all()
