@@ -2540,9 +2540,7 @@ __device__ __noinline__ uint32_t deep_mid(const SampleArgs& a, Shared& S, int64_
   const int n_reg = (int)S.deep_n;
   const double vf = (double)key_f32(thr) / T;  // the region floor's value
   const double vfc = vf * ((double)kDeepBins / kDeepSpan);
-  // the largest float below the floor's logit: l <= l_below iff f32_key(l) < thr
-  // (NaN aside; -0 and +0 share a key, and the float below both is -2^-149)
-  const float l_below = key_f32(thr - 1u);
+  const float l_below = key_below(thr);  // the largest logit below the floor's
   uint64_t* mass = S.sorted;  // [kDeepBins - 1] terms in units of 2^-40 e^(c_b - M)
   // specials: out with their raw values (where pass 1 counted them; the
   // same units, so exactly), in with their penalised ones below the floor
@@ -2983,7 +2981,7 @@ __device__ __noinline__ uint32_t deep_draw(const SampleArgs& a, FinishLds& U) {
   const int n_sp = (int)(S.n_special < (uint32_t)kSpecialCap ? S.n_special : (uint32_t)kSpecialCap);
   const double rT = 1.0 / T;
   const double vfc = (double)key_f32(S.deep_thr) / T * ((double)kDeepBins / kDeepSpan);
-  const float l_below = key_f32(S.deep_thr - 1u);
+  const float l_below = key_below(S.deep_thr);
   deep_setup(S, n_sp, true);
   // ---- pass 1: the tail's mass per bin
   const double tail = deep_histogram(a, row, cfg.softcap, T, rT, S.deep_m, l_below, vfc, S.sorted, S.tab);
@@ -3166,7 +3164,7 @@ __device__ __noinline__ void deep1_part(const SampleArgs& a, Shared& S, int64_t 
   const double M = D.M;
   const uint32_t thr = D.thr;
   const double vfc = (double)key_f32(thr) / T * ((double)kDeepBins / kDeepSpan);
-  const float l_below = key_f32(thr - 1u);
+  const float l_below = key_below(thr);
   uint64_t* mass = S.sorted;
   GS_CHECK_RESET();
   for (int b = tid; b < kDeepBins; b += kFinishThreads) mass[GS_CK(b, kFinishCap)] = 0ull;

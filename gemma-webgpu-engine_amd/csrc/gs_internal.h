@@ -68,6 +68,12 @@ __host__ __device__ __forceinline__ float key_f32(uint32_t k) {
   const uint32_t b = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
   return __builtin_bit_cast(float, b);
 }
+// The largest float whose key lies below k: l <= key_below(k) iff f32_key(l) < k
+// (NaN aside). The two zeros share a key, so below theirs comes -2^-149: the
+// key between, which no value has, reads as -0. (k = 0: NaN, below nothing.)
+__host__ __device__ __forceinline__ float key_below(uint32_t k) {
+  return k == 0x80000000u ? -0x1p-149f : key_f32(k - 1u);
+}
 // 64-bit key of an f64 value (same conventions).
 __host__ __device__ __forceinline__ uint64_t f64_key(double x) {
   uint64_t b = __builtin_bit_cast(uint64_t, x);

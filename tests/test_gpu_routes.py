@@ -390,3 +390,44 @@ def test_full_vocabulary_draw_within_the_scan_margin(sampler, oracle, n_hist):
         check(gs, oracle, "scan margin", out, [x] * len(us), hists, cfgs, us)
         exact = (out.flags & gs.GS_FLAG_EXACT_PATH) != 0
         assert np.array_equal(exact, np.array(near)), (hints, list(zip(us, exact)))
+
+
+@pytest.mark.parametrize("n_hist", [0, 30])
+def test_full_vocabulary_draws_with_a_zero_floor(oracle, n_hist):
+    """Rows whose candidate lists end at zeros of both signs (every wave's
+    16th lane maximum is 0), drawn past the lists and within the scan
+    normaliser's margin of a prefix sum: the deep draw's tail starts below
+    the zeros, which its candidates hold already."""
+    import torch
+
+    gs = _gs()
+    Vs, T = 3 * 8192, 0.8
+    rng = np.random.default_rng(31)
+    rows, hists, cfgs, us = [], [], [], []
+    for r in range(12):
+        x = np.minimum(rng.normal(-2, 1, Vs), -0.01)
+        ids = rng.permutation(Vs)
+        x[ids[:120]] = np.round(rng.uniform(0.25, 3, 120) * 8) / 8
+        x[ids[120:600]] = 0.0
+        x[ids[120:600:2]] = -0.0
+        x = x.astype(np.float32)
+        hist = ids[:600:600 // n_hist].tolist() if n_hist else []
+        v = x.astype(np.float64)
+        for i in hist:
+            v[i] = v[i] / 1.2 if v[i] >= 0 else v[i] * 1.2
+        e = np.sort(np.exp(v / T))[::-1]
+        cum = np.cumsum(e / e.sum())
+        rows.append(x)
+        hists.append(hist)
+        cfgs.append(gs.DecodingConfig(temperature=T, topK=0, topP=1.0, repetitionPenalty=1.2 if n_hist else 1.0,
+                                      repetitionWindow=64 if n_hist else 0))
+        us.append(float(cum[100] + 1e-7 if r % 3 == 0 else cum[610] + rng.random() * (1 - cum[610])))
+    s = gs.Sampler(vocab_size=Vs, max_rows=16)
+    try:
+        conf = np.stack([gs.runtime.row_config(c, uniform=u) for c, u in zip(cfgs, us)])
+        for hints in (None, 0):
+            out = s.sample(torch.from_numpy(np.stack(rows)).cuda(), conf, histories=hists, hints=hints)
+            assert not (out.flags & gs.GS_FLAG_EXACT_PATH).any(), out.flags
+            check(gs, oracle, "zero floor", out, rows, hists, cfgs, us)
+    finally:
+        s.close()
