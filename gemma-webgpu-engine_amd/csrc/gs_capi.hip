@@ -284,13 +284,13 @@ hipError_t launch_sample(const Workspace& w, const gs_batch* b, hipStream_t s, c
   if (e != hipSuccess) return e;
   if (deep) {
     // rows queued by the finish kernel for the multi-workgroup deep draw
-    launch_deep(a, s, ev[GS_STAGE_DEEP]);
+    launch_deep(a, s, LaunchEvents{ev[GS_STAGE_DEEP].start, a.typical ? nullptr : ev[GS_STAGE_DEEP].stop});
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   if (a.typical) {
     // the typical-p rows that the finish left
-    launch_typical(a, s);
+    launch_typical(a, s, LaunchEvents{deep ? nullptr : ev[GS_STAGE_DEEP].start, ev[GS_STAGE_DEEP].stop});
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -572,7 +572,7 @@ int gs_sample(gs_context* ctx, const gs_batch* b, void* stream) {
   const int32_t slot = timing_slot(ctx);
   LaunchEvents ev[GS_STAGE_COUNT];
   for (int k = GS_STAGE_SCAN; k <= GS_STAGE_FINISH; ++k) ev[k] = stage_events(ctx, slot, k);
-  if (deep_launch(w, b)) ev[GS_STAGE_DEEP] = stage_events(ctx, slot, GS_STAGE_DEEP);
+  if (deep_launch(w, b) || (b->hints & GS_BATCH_TYPICAL)) ev[GS_STAGE_DEEP] = stage_events(ctx, slot, GS_STAGE_DEEP);
   if (b->rows > ctx->exact_slots) ev[GS_STAGE_EXACT] = stage_events(ctx, slot, GS_STAGE_EXACT);
   const hipError_t e = launch_sample(w, b, pick_stream(ctx, stream), ev);
   if (e != hipSuccess) return fail(ctx, GS_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
@@ -1056,7 +1056,7 @@ int gs_lmhead_sample(gs_context* ctx, const void* hidden, const void* weight, in
   const int32_t slot = timing_slot(ctx);
   LaunchEvents ev[GS_STAGE_COUNT];
   for (int k = GS_STAGE_LMHEAD; k <= GS_STAGE_FINISH; ++k) ev[k] = stage_events(ctx, slot, k);
-  if (deep_launch(w, &b)) ev[GS_STAGE_DEEP] = stage_events(ctx, slot, GS_STAGE_DEEP);
+  if (deep_launch(w, &b) || (b.hints & GS_BATCH_TYPICAL)) ev[GS_STAGE_DEEP] = stage_events(ctx, slot, GS_STAGE_DEEP);
   if (b.rows > ctx->exact_slots) ev[GS_STAGE_EXACT] = stage_events(ctx, slot, GS_STAGE_EXACT);
   hipStream_t s = pick_stream(ctx, stream);
   launch_lmhead_scan((const uint16_t*)hidden, (const uint16_t*)weight, b.rows, width, softcap, logits_scratch,

@@ -594,7 +594,7 @@ void launch_exp2_check(uint32_t first, uint32_t count, unsigned long long* worst
 void launch_finish(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
 void launch_exact(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
 void launch_deep(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
-void launch_typical(const SampleArgs& a, hipStream_t s);
+void launch_typical(const SampleArgs& a, hipStream_t s, LaunchEvents ev = {});
 // partial: logprob_bytes() of device memory
 size_t logprob_bytes();
 void launch_logprob(const void* logits, int32_t dtype, int32_t rows, int64_t stride, int32_t vocab,

@@ -455,10 +455,10 @@ __global__ __launch_bounds__(kTypThreads) void typical_kernel(SampleArgs) {
 
 }  // namespace
 
-void launch_typical(const SampleArgs& a, hipStream_t s) {
+void launch_typical(const SampleArgs& a, hipStream_t s, LaunchEvents ev) {
   const dim3 grid(a.rows), block(kTypThreads);
-  if (a.dtype == GS_BF16) hipLaunchKernelGGL(typical_kernel<uint16_t>, grid, block, 0, s, a);
-  else hipLaunchKernelGGL(typical_kernel<float>, grid, block, 0, s, a);
+  if (a.dtype == GS_BF16) hipExtLaunchKernelGGL(typical_kernel<uint16_t>, grid, block, 0, s, ev.start, ev.stop, 0, a);
+  else hipExtLaunchKernelGGL(typical_kernel<float>, grid, block, 0, s, ev.start, ev.stop, 0, a);
 }
 
 }  // namespace gs

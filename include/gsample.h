@@ -342,7 +342,8 @@ int gs_check_exp2(gs_context* ctx, float lo, float hi, double* max_rel_err, floa
 #define GS_STAGE_SCAN 1   /* scan_kernel: the one HBM pass over the logits */
 #define GS_STAGE_FINISH 2 /* finish_kernel: per-row merge, filters and draw */
 #define GS_STAGE_EXACT 3  /* exact_kernel: replay of rows beyond the context's exact slots */
-#define GS_STAGE_DEEP 4   /* deep1_kernel .. deep_final_kernel: full-vocabulary draws over many workgroups */
+#define GS_STAGE_DEEP 4   /* deep1_kernel .. deep_final_kernel: full-vocabulary draws over many workgroups,
+                             and typical_kernel: typical-p over the whole vocabulary */
 #define GS_STAGE_COUNT 5
 int gs_timing_begin(gs_context* ctx, int32_t max_calls);
 int gs_timing_end(gs_context* ctx, double* stage_ms, int32_t* calls);

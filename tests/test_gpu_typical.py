@@ -265,3 +265,31 @@ def test_typical_rows_are_decided_once(oracle, V):
         assert np.array_equal(out.flags, plain.flags) and np.array_equal(out.probabilities, plain.probabilities)
     else:
         assert (plain.flags & gs.GS_FLAG_EXACT_PATH).all() and not (out.flags & gs.GS_FLAG_EXACT_PATH).all()
+
+
+def test_typical_launch_is_timed():
+    """The typical-p kernel's time is in the deep stage, alone and after full-vocabulary draws."""
+    import torch
+
+    import gsample as gs
+
+    V = 50000
+    x = torch.from_numpy(np.random.default_rng(3).normal(0, 3, (8, V)).astype(np.float32)).cuda()
+    draw = gs.DecodingConfig(temperature=0.8, topK=0, topP=1.0, typicalP=1.0, repetitionPenalty=1.0, repetitionWindow=0)
+    s = gs.Sampler(vocab_size=V, max_rows=8)
+    try:
+        for n in (0, 4, 8):  # typical-p rows among full-vocabulary draws
+            conf = np.stack([gs.runtime.row_config(draw.merged(typicalP=0.9 if i < n else 1.0), uniform=0.3)
+                             for i in range(8)])
+            b, keep = s.prepare(x, conf)
+            want = (gs.runtime.GS_BATCH_TYPICAL if n else 0) | (gs.runtime.GS_BATCH_FULL_DRAWS if n < 8 else 0)
+            assert b.hints == want
+            s.launch(b)
+            s.synchronize()
+            s.timing_begin(3)
+            for _ in range(3):
+                s.launch(b)
+            ms, calls = s.timing_end()["deep"]
+            assert calls == 3 and ms > 3 * (0.03 if n else 0.0), (n, ms, calls)
+    finally:
+        s.close()
