@@ -41,6 +41,8 @@ struct gs_context {
   std::vector<int32_t> next;      // viability folded in
   std::vector<uint8_t> finals;
   std::vector<uint8_t> viable;
+  std::vector<int64_t> first_bytes;  // tokens by their first byte
+  std::vector<double> live_share;    // per state: share of the vocabulary whose first byte it takes
   int32_t* d_states = nullptr;
   int32_t states_cap = 0;
   // device staging for the host-array entry points (grown on demand)
@@ -824,6 +826,20 @@ int gs_check_exp2(gs_context* ctx, float lo, float hi, double* max_rel_err, floa
   return GS_OK;
 }
 
+// live_share from the vocabulary's first bytes and the DFA (both set).
+static void count_live(gs_context* ctx) {
+  ctx->live_share.assign(ctx->next.size() / 256, 0.0);
+  if (ctx->first_bytes.empty()) return;
+  for (size_t s = 0; s < ctx->live_share.size(); ++s) {
+    int64_t live = 0;
+    for (int c = 0; c < 256; ++c) {
+      const int32_t t = ctx->next[s * 256 + c];
+      if (t >= 0 && ctx->viable[t]) live += ctx->first_bytes[c];
+    }
+    ctx->live_share[s] = (double)live / ctx->vocab;
+  }
+}
+
 int gs_set_vocab(gs_context* ctx, const int64_t* offsets, const uint8_t* bytes, int64_t n_bytes) {
   if (!ctx || !offsets || (n_bytes > 0 && !bytes) || n_bytes < 0) return fail(ctx, GS_ERR_INVALID_ARGUMENT, "bad vocab");
   const int64_t V = ctx->vocab;
@@ -842,6 +858,10 @@ int gs_set_vocab(gs_context* ctx, const int64_t* offsets, const uint8_t* bytes, 
   GS_HIP(ctx, hipMalloc(&ctx->d_vocab_bytes, std::max<int64_t>(n_bytes, 16)));
   GS_HIP(ctx, hipMemcpy(ctx->d_vocab_offsets, offsets, sizeof(int64_t) * (V + 1), hipMemcpyHostToDevice));
   if (n_bytes) GS_HIP(ctx, hipMemcpy(ctx->d_vocab_bytes, bytes, n_bytes, hipMemcpyHostToDevice));
+  ctx->first_bytes.assign(256, 0);
+  for (int64_t t = 0; t < V; ++t)
+    if (offsets[t + 1] > offsets[t]) ctx->first_bytes[bytes[offsets[t]]]++;
+  count_live(ctx);
   return GS_OK;
 }
 
@@ -880,6 +900,7 @@ int gs_set_dfa(gs_context* ctx, int32_t n_states, const int32_t* next, const uin
   ctx->n_states = n_states;
   ctx->finals.assign(finals, finals + n_states);
   ctx->viable = viable;
+  count_live(ctx);
   return GS_OK;
 }
 
@@ -900,8 +921,10 @@ int gs_build_masks(gs_context* ctx, const int32_t* states, int32_t n, uint32_t* 
     ctx->states_cap = n;
   }
   GS_HIP(ctx, hipMemcpyAsync(ctx->d_states, states, sizeof(int32_t) * n, hipMemcpyHostToDevice, s));
-  launch_masks(ctx->d_vocab_offsets, ctx->d_vocab_bytes, ctx->vocab, ctx->d_next, ctx->d_states, n, mask_table,
-               ctx->mask_words, ctx->n_states, s);
+  double share = 0.0;
+  for (int32_t i = 0; i < n; ++i) share += ctx->live_share[states[i]];
+  launch_masks(ctx->d_vocab_offsets, ctx->d_vocab_bytes, ctx->vocab, ctx->d_next, ctx->d_states, n, share / n,
+               mask_table, ctx->mask_words, ctx->n_states, s);
   GS_HIP(ctx, hipGetLastError());
   GS_HIP(ctx, hipStreamSynchronize(s));  // the state list is reused by the next call
   return GS_OK;

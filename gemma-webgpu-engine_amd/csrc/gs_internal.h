@@ -601,8 +601,8 @@ void launch_logprob(const void* logits, int32_t dtype, int32_t rows, int64_t str
                     const int32_t* tokens, double* out, void* partial, int32_t cu_count, hipStream_t s);
 void launch_mask_logits(const float* raw, int64_t n, const int32_t* ids, int64_t n_ids, float* out, hipStream_t s);
 void launch_masks(const int64_t* offsets, const uint8_t* bytes, int32_t vocab, const int16_t* next,
-                  const int32_t* states, int32_t n, uint32_t* masks, int32_t mask_words, int32_t n_states,
-                  hipStream_t s);
+                  const int32_t* states, int32_t n, double share, uint32_t* masks, int32_t mask_words,
+                  int32_t n_states, hipStream_t s);
 void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* words, int32_t block_major,
                        const float* scales, int32_t V, double in_scale, double out_scale, float* out,
                        int32_t cu_count, hipStream_t s, LaunchEvents ev = {});

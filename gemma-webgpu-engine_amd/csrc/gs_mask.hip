@@ -31,6 +31,56 @@ constexpr int kMaskWaves = kMaskThreads / 64;
 constexpr int kMaskStates = 64;  // requested states walked together, a bit each
 constexpr int kLdsStates = 192;  // tables up to 192 x 256 x int16 (96 KiB) stay in LDS
 
+// A token's first 16 bytes (past its end its last one again).
+__device__ __forceinline__ void token_bytes(const uint8_t* bytes, int64_t b0, int len, uint64_t* lo, uint64_t* hi) {
+  *lo = *hi = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint64_t v = len > 0 ? bytes[b0 + (i < len ? i : len - 1)] : 0u;
+    if (i < 8) *lo |= v << (8 * i);
+    else *hi |= v << (8 * (i - 8));
+  }
+}
+
+constexpr int kWalkThreads = 256;
+constexpr int kWalkLdsStates = 96;  // tables up to 48 KiB
+constexpr int kWalkLdsVocab = 196608;
+
+// Every token walked from each requested state in turn, a wave waiting for
+// its longest lane (launch_masks says where this is the faster kernel).
+template <bool kInLds>
+__global__ __launch_bounds__(kWalkThreads) void walk_masks_kernel(const int64_t* offsets, const uint8_t* bytes,
+                                                                  int32_t vocab, const int16_t* next,
+                                                                  int32_t n_states, const int32_t* states, int32_t n,
+                                                                  uint32_t* masks, int32_t mask_words) {
+  __shared__ uint4 s_next[kInLds ? kWalkLdsStates * 32 : 1];
+  const int lane = threadIdx.x & 63;
+  const int64_t t = (int64_t)blockIdx.x * kWalkThreads + threadIdx.x;
+  int64_t b0 = 0, b1 = 0;
+  if (t < vocab) { b0 = offsets[t]; b1 = offsets[t + 1]; }
+  const int len = (int)(b1 - b0);
+  uint64_t lo, hi;
+  token_bytes(bytes, b0, len, &lo, &hi);
+  if (kInLds) {
+    for (int i = threadIdx.x; i < n_states * 32; i += kWalkThreads) s_next[i] = ((const uint4*)next)[i];
+    __syncthreads();
+  }
+  const int16_t* table = kInLds ? (const int16_t*)s_next : next;
+  const int64_t word = ((t & ~63ll) >> 5) + lane;
+  for (int q = 0; q < n; ++q) {
+    int32_t s = states[q];
+    bool legal = len > 0 && s >= 0 && s < n_states;
+    for (int i = 0; legal && i < len; ++i) {
+      const uint32_t b = i < 8 ? (uint32_t)(lo >> (8 * i)) & 0xFFu
+                               : (i < 16 ? (uint32_t)(hi >> (8 * (i - 8))) & 0xFFu : bytes[b0 + i]);
+      s = table[s * 256 + (int)b];
+      legal = s >= 0;
+    }
+    const uint64_t bits = __ballot(legal);
+    if (lane < 2 && word < mask_words) masks[(int64_t)q * mask_words + word] = (uint32_t)(bits >> (32 * lane));
+  }
+}
+
 struct MaskLds {
   int16_t next[kLdsStates * 256];
   int16_t first[256][kMaskStates + 2];       // the state after a token's first byte (rows a bank apart)
@@ -61,13 +111,8 @@ __global__ __launch_bounds__(kMaskThreads) void build_masks_kernel(const int64_t
     for (int i = tid; i < n_states * 32; i += kMaskThreads) ((uint4*)L.next)[i] = ((const uint4*)next)[i];
   }
   // the first 16 bytes in registers, the rest read on demand
-  uint64_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint64_t v = len > 0 ? bytes[b0 + (i < len ? i : len - 1)] : 0u;
-    if (i < 8) lo |= v << (8 * i);
-    else hi |= v << (8 * (i - 8));
-  }
+  uint64_t lo, hi;
+  token_bytes(bytes, b0, len, &lo, &hi);
   __syncthreads();
   const int16_t* table = kInLds ? L.next : next;
   for (int q0 = 0; q0 < n; q0 += kMaskStates) {
@@ -310,17 +355,33 @@ void launch_mask_logits(const float* raw, int64_t n, const int32_t* ids, int64_t
   }
 }
 
+// share: of the vocabulary, by first byte, that the requested states take on
+// average. The walk of every token is the faster kernel for few states and
+// where first bytes rule out little; its line depends on whether its table is
+// in LDS (1.2 times the speed, up to 96 states, and a loss past about 200000
+// tokens, where the 48 KiB cost resident waves). Whole calls in us, walk |
+// by first bytes: 32000 tokens, 8 states, share 0.3: 25 | 30 for 8 requested,
+// 67 | 64 for 64; share 0.8: 105 | 169 for 64. 262144 tokens, 300 states, share
+// 0.3: 29 | 29 for 8 requested, 38 | 32 for 16; for 64 requested 168 | 141 at
+// share 0.8, 177 | 217 at share 1. With one state 21 | 25 on either.
 void launch_masks(const int64_t* offsets, const uint8_t* bytes, int32_t vocab, const int16_t* next,
-                  const int32_t* states, int32_t n, uint32_t* masks, int32_t mask_words, int32_t n_states,
-                  hipStream_t s) {
-  const dim3 grid((vocab + kMaskThreads - 1) / kMaskThreads), block(kMaskThreads);
-  if (n_states <= kLdsStates) {
-    hipLaunchKernelGGL(build_masks_kernel<true>, grid, block, 0, s, offsets, bytes, vocab, next, n_states, states, n,
-                       masks, mask_words);
+                  const int32_t* states, int32_t n, double share, uint32_t* masks, int32_t mask_words,
+                  int32_t n_states, hipStream_t s) {
+#define GS_MASKS(kernel, threads)                                                                               \
+  hipLaunchKernelGGL(kernel, dim3((vocab + threads - 1) / threads), dim3(threads), 0, s, offsets, bytes, vocab, \
+                     next, n_states, states, n, masks, mask_words)
+  const bool walk_lds = n_states <= kWalkLdsStates && vocab <= kWalkLdsVocab;
+  const int few = walk_lds ? 16 : (vocab > kWalkLdsVocab ? 8 : 10);
+  const double most = walk_lds ? (n_states < 32 ? 0.6 : 0.66) : 0.8;
+  if (n < few || share > most) {
+    if (walk_lds && n >= 4) GS_MASKS(walk_masks_kernel<true>, kWalkThreads);
+    else GS_MASKS(walk_masks_kernel<false>, kWalkThreads);
+  } else if (n_states <= kLdsStates) {
+    GS_MASKS(build_masks_kernel<true>, kMaskThreads);
   } else {
-    hipLaunchKernelGGL(build_masks_kernel<false>, grid, block, 0, s, offsets, bytes, vocab, next, n_states, states, n,
-                       masks, mask_words);
+    GS_MASKS(build_masks_kernel<false>, kMaskThreads);
   }
+#undef GS_MASKS
 }
 
 template <typename In>
