@@ -3,7 +3,7 @@
 //
 // The reference's producer is an int2 QAT GEMV (src/webgpu/decode-lm-head.ts:
 // 187-340); this is the bf16 tied-embedding variant the sampler consumes.
-// Two kernels, one order of sums: the K blocks of a row (64 wide) fall into
+// Two kernels, one order of sums: the K steps of a row (32 wide) fall into
 // eight ranges, each summed by v_mfma_f32_16x16x32_bf16 in K order, and the
 // ranges are added one by one in binary32, so a logit is the same bits
 // whichever kernel and batch it comes from (and about half the rounding error
@@ -102,16 +102,30 @@ __device__ __forceinline__ void gemm_fetch(Rsrc r, char* lds, const uint32_t (&o
 #endif
 }
 
+// The running tiles into the totals, at the end of a range of K.
+template <int kMT>
+__device__ __forceinline__ void gemm_flush(f32x4 (&acc)[4][kMT], f32x4 (&total)[4][kMT]) {
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+#pragma unroll
+    for (int b = 0; b < kMT; ++b) {
+      total[a][b] += acc[a][b];
+      acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+}
+
 // One K block: the next fetches go out, then two K-32 steps of this wave's
-// 4 x kMT tiles; `flush` (uniform) then moves the running tiles into the
-// totals. The buffers are distinct objects, so the compiler's own waits
-// before the reads cover nothing that is still being fetched.
-template <int kMT, typename Rsrc>
+// 4 x kMT tiles; a range ends (uniform) after the second step or, with
+// kHalf, also after the first. The buffers are distinct objects, so the
+// compiler's own waits before the reads cover nothing that is still being
+// fetched.
+template <int kMT, bool kHalf, typename Rsrc>
 __device__ __forceinline__ void gemm_block(const char* __restrict__ w, const char* __restrict__ h,
                                            char* __restrict__ w_next, char* __restrict__ h_next,
                                            Rsrc wr, Rsrc hr,
                                            const uint32_t (&w_off)[4], const uint32_t (&h_off)[kMT], uint32_t w_k,
-                                           uint32_t h_k, const uint32_t (&pos)[2], bool flush,
+                                           uint32_t h_k, const uint32_t (&pos)[2], bool half_flush, bool flush,
                                            f32x4 (&acc)[4][kMT], f32x4 (&total)[4][kMT]) {
   gemm_fetch<kMT>(hr, h_next, h_off, h_k);
   asm volatile("" ::: "memory");  // W's fetches stay the last four issued
@@ -132,20 +146,17 @@ __device__ __forceinline__ void gemm_block(const char* __restrict__ w, const cha
       for (int b = 0; b < kMT; ++b)
         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][a], hf[s][b], acc[a][b], 0, 0, 0);
     }
+    if (kHalf && s == 0 && half_flush) gemm_flush<kMT>(acc, total);
   }
-  if (flush) {
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-#pragma unroll
-      for (int b = 0; b < kMT; ++b) {
-        total[a][b] += acc[a][b];
-        acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      }
-    }
-  }
+  if (flush) gemm_flush<kMT>(acc, total);
 }
 
-template <int kMT>  // 16-row tiles of H per wave: 32 kMT rows of H per workgroup
+// kMT: 16-row tiles of H per wave (32 kMT rows of H per workgroup). kHalf:
+// the resident kernel's ranges at widths off 512, which may end within a K
+// block; where that kernel never runs they end with blocks (the flush between
+// a block's steps costs up to 3%, and ranges of whole blocks would cost the
+// resident kernel up to 6% there: V 32000, D 576, one row 15.9 us | 15.0).
+template <int kMT, bool kHalf>
 __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint16_t* __restrict__ H,
                                                                       const uint16_t* __restrict__ W, int M, int D,
                                                                       int V, int m_blocks, int wide, float cap,
@@ -196,10 +207,13 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
     }
   }
   const int nk = D / kGemmK;
-  int range = 0, bound = 0;  // `bound`: the block that ends the current range (empty ranges are passed over)
+  int range = 0, bound = 0;  // `bound`: the K step that ends the current range (empty ranges are passed over)
   auto next_bound = [&]() __attribute__((always_inline)) {
     const int done = bound;
-    do { bound = ++range * nk / kGemmChunks; } while (bound == done && range < kGemmChunks);
+    do {
+      ++range;
+      bound = kHalf ? range * 2 * nk / kGemmChunks : 2 * (range * nk / kGemmChunks);
+    } while (bound == done && range < kGemmChunks);
   };
   next_bound();
   const int first = lmhead_first_range(v0, D) * (nk / kGemmChunks);  // blocks wrap around after the last
@@ -211,10 +225,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
     // block kb's rows have landed for every wave (W's block kb + 1, fetched
     // after them, may still be under way), and every wave has read block kb - 1
     asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const bool flush = kb + 1 == bound;
+    const bool half_flush = kHalf && 2 * kb + 1 == bound;
+    if (half_flush) next_bound();
+    const bool flush = 2 * kb + 2 == bound;
     if (flush) next_bound();
-    gemm_block<kMT>(w + w_src, h + h_src, wn + w_dst, hn + h_dst, wr, hr, w_off, h_off, at(kb + 2), at(kb + 1), pos,
-                    flush, acc, total);
+    gemm_block<kMT, kHalf>(w + w_src, h + h_src, wn + w_dst, hn + h_dst, wr, hr, w_off, h_off, at(kb + 2), at(kb + 1),
+                           pos, half_flush, flush, acc, total);
   };
   gemm_fetch<4>(wr, sw0 + w_dst, w_off, at(0));
   gemm_fetch<kMT>(hr, sh0 + h_dst, h_off, at(0));
@@ -277,8 +293,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
 // D 2048) dealt round-robin to the workgroups, so the chip reads a window of
 // adjacent runs at a time (199 us against 203 us for one contiguous range
 // per workgroup).
-//   * 8 waves split K: wave w owns the 64-wide K blocks [w nB / 8, (w+1) nB / 8)
-//     of the nB = D / 64, its H slice (64 rows) held as MFMA A operands
+//   * 8 waves split K: wave w owns the 32-wide K steps [w nS / 8, (w+1) nS / 8)
+//     of the nS = D / 32, its H slice (64 rows) held as MFMA A operands
 //     (v_mfma_f32_16x16x32_bf16: lane i + 16 g holds k = 32 s + 8 g .. + 7 of
 //     row i of an M tile, 4 M tiles);
 //   * per step a lane loads 16 bytes per K step of one vocabulary row (the
@@ -308,7 +324,7 @@ constexpr int32_t kResNT = 2;     // non-temporal cache policy of the streams
 constexpr int kResStage = 16;     // steps of logits staged per flush
 constexpr int kResStageStride = kResStage * kResN + 4;  // LDS floats per staged row
 
-template <int kS>  // K steps per wave: 2, 4, 6 or 8
+template <int kS>  // K steps per wave, at most 8
 __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint16_t* __restrict__ H,
                                                                       const uint16_t* __restrict__ W, int M, int D,
                                                                       int V, float cap, float* __restrict__ out) {
@@ -316,9 +332,9 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
   __shared__ __attribute__((aligned(16))) float stage[64 * kResStageStride];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 15, g = lane >> 4;
-  const int n_blocks = D / 64;
-  const int s_lo = 2 * (wave * n_blocks / kResWaves), s_hi = 2 * ((wave + 1) * n_blocks / kResWaves);
-  const int my_steps = s_hi - s_lo;  // kS or kS - 2
+  const int n_steps = D / 32;
+  const int s_lo = wave * n_steps / kResWaves, s_hi = (wave + 1) * n_steps / kResWaves;
+  const int my_steps = s_hi - s_lo;  // kS or kS - 1
   // this workgroup's steps k = 0 .. k_end - 1: run blockIdx.x + gridDim.x r
   // (r = k / kResStage), tile kResStage run + k % kResStage of 16 vocabulary
   // rows; steps on tiles past the last are empty
@@ -432,10 +448,11 @@ __global__ __launch_bounds__(kResThreads) void lmhead_resident_kernel(const uint
 
 void launch_lmhead(const uint16_t* hidden, const uint16_t* weight, int32_t m, int32_t width, int32_t vocab,
                    float softcap, float* out, int32_t cu_count, hipStream_t s, LaunchEvents ev) {
-  if (width <= kResMaxWidth && width % 32 == 0 && m <= kResM && vocab % 4 == 0 && ((uintptr_t)out & 15) == 0 &&
-      (int64_t)vocab * kResM * 4 < ((int64_t)1 << 31)) {
+  const bool resident = width <= kResMaxWidth && width % 32 == 0 && vocab % 4 == 0 &&
+                        (int64_t)vocab * kResM * 4 < ((int64_t)1 << 31);
+  if (resident && m <= kResM && ((uintptr_t)out & 15) == 0) {
     // one workgroup per compute unit
-    const int k_steps = 2 * ((width / 64 + kResWaves - 1) / kResWaves);
+    const int k_steps = (width / 32 + kResWaves - 1) / kResWaves;
     const dim3 grid(cu_count > 0 ? cu_count : 256), block(kResThreads);
     switch (k_steps) {
 #define GS_RES_CASE(k)                                                                                               \
@@ -443,9 +460,13 @@ void launch_lmhead(const uint16_t* hidden, const uint16_t* weight, int32_t m, in
     hipExtLaunchKernelGGL(lmhead_resident_kernel<k>, grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m,     \
                           width, vocab, softcap, out);                                                               \
     break;
+      GS_RES_CASE(1)
       GS_RES_CASE(2)
+      GS_RES_CASE(3)
       GS_RES_CASE(4)
+      GS_RES_CASE(5)
       GS_RES_CASE(6)
+      GS_RES_CASE(7)
       GS_RES_CASE(8)
 #undef GS_RES_CASE
     }
@@ -457,16 +478,20 @@ void launch_lmhead(const uint16_t* hidden, const uint16_t* weight, int32_t m, in
   const int v_tiles = (vocab + kGemmV - 1) / kGemmV;
   const dim3 grid((unsigned)((v_tiles + 7) / 8 * 8 * m_blocks)), block(kGemmThreads);
   const int wide = vocab % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  switch (tiles) {
-#define GS_GEMM_CASE(k)                                                                                               \
-  case k:                                                                                                             \
-    hipExtLaunchKernelGGL(lmhead_gemm_kernel<k>, grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m, width,   \
-                          vocab, m_blocks, wide, softcap, out);                                                       \
+  switch (resident && width % 512 != 0 ? -tiles : tiles) {
+#define GS_GEMM_CASE(n, k, half)                                                                                       \
+  case n:                                                                                                              \
+    hipExtLaunchKernelGGL((lmhead_gemm_kernel<k, half>), grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m,   \
+                          width, vocab, m_blocks, wide, softcap, out);                                                 \
     break;
-    GS_GEMM_CASE(1)
-    GS_GEMM_CASE(2)
-    GS_GEMM_CASE(3)
-    GS_GEMM_CASE(4)
+    GS_GEMM_CASE(1, 1, false)
+    GS_GEMM_CASE(2, 2, false)
+    GS_GEMM_CASE(3, 3, false)
+    GS_GEMM_CASE(4, 4, false)
+    GS_GEMM_CASE(-1, 1, true)
+    GS_GEMM_CASE(-2, 2, true)
+    GS_GEMM_CASE(-3, 3, true)
+    GS_GEMM_CASE(-4, 4, true)
 #undef GS_GEMM_CASE
   }
 }

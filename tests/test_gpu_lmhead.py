@@ -158,6 +158,10 @@ def test_lmhead_shapes_match_f64(vocab, width, m):
     (2052, 576, 129, 0),   # nine blocks over eight ranges; two row blocks
     (1028, 1024, 257, 0),  # three row blocks
     (4100, 2048, 128, 1),  # logits 4 bytes off a 16-byte address
+    (2052, 576, 30, 1),    # the same, one- and two-tile blocks, ranges that end within a K block
+    (2052, 1984, 60, 1),
+    (1028, 192, 70, 0),    # ranges of one step, two in a K block
+    (1027, 576, 100, 0),   # no resident kernel at this vocabulary: ranges of whole blocks
     (127, 2048, 33, 0),    # less than one slab, odd rows
     (2049, 3840, 1, 0),    # wide, odd, one row
 ])
@@ -186,8 +190,8 @@ def test_lmhead_gemm_edges(vocab, width, m, shift):
             err_bound = bound + (4 * np.spacing(np.abs(exp).astype(np.float32)).astype(np.float64) if cap > 0 else 0)
             assert np.all(np.abs(got - exp) <= err_bound), (cap, float((np.abs(got - exp) / err_bound).max()))
             assert bool((out[m:] == 7.0).all()) and bool((store[:shift] == 7.0).all())
-            if vocab % 4 == 0 and width <= 2048 and m > 64:
+            if vocab % 4 == 0 and width <= 2048 and (m > 64 or shift):
                 alone = s.lmhead(hidden[:64].contiguous(), weight, softcap_value=cap)
-                assert torch.equal(alone, out[:64])
+                assert torch.equal(alone, out[:min(m, 64)])
     finally:
         s.close()
