@@ -42,7 +42,8 @@ namespace gs {
 namespace {
 
 constexpr int kQatThreads = 256;
-constexpr int kQatLdsDoubles = 4096;  // activations staged per pass: rows x width <= 32 KiB
+constexpr int kQatLdsDoubles = 4096;  // activations staged: one row of width 4096 or two of 2048
+constexpr int64_t kQatSmall = 60000000;  // products of one or two rows
 
 struct QatArgs {
   const float* x;         // [M][D]
@@ -178,18 +179,17 @@ constexpr int kQatTileWaves = kQatTileThreads / 64;
 constexpr int32_t kQatNT = 2;        // non-temporal cache policy of the code stream
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Rows 2 tile and 2 tile + 1 of x, one launch, one workgroup per compute unit
-// over a contiguous run of 16-row vocabulary tiles. Each workgroup checks the
-// two rows and writes their limbs into LDS as a 16-row operand tile (rows
-// 8 r + limb, limb 7 zero; one thread per code word of 16 activations); its
-// 16 waves then take the run's tiles in turn, the next tile's codes loading
-// while the current one multiplies. A row the check refused takes the
-// binary64 path over the same vocabulary rows afterwards. (Four 256-thread
-// workgroups per compute unit, each repeating the check and the limbs, took
-// 25.3 us instead of 24.4 at V 262144, D 1536; reducing the check's sums
-// through an LDS array by one wave per row instead of LDS atomics, 24.9 us
-// instead of 24.0.)
-__global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, int32_t tile) {
+// One or two rows of x, one workgroup per compute unit over a contiguous run
+// of 16-row vocabulary tiles. Each workgroup checks the rows and writes their
+// limbs into LDS as a 16-row operand tile (rows 8 r + limb, limb 7 zero; one
+// thread per code word of 16 activations); its 16 waves then take the run's
+// tiles in turn, the next tile's codes loading while the current one
+// multiplies. A row the check refused takes the binary64 path over the same
+// vocabulary rows afterwards. (Four 256-thread workgroups per compute unit,
+// each repeating the check and the limbs, took 25.3 us instead of 24.4 at
+// V 262144, D 1536; reducing the check's sums through an LDS array by one wave
+// per row instead of LDS atomics, 24.9 us instead of 24.0.)
+__global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a) {
   __shared__ union __attribute__((aligned(16))) {
     i32x4 op[kQatMaxSteps][64];   // the integer path's operand tile
     double act[2 * 2048];         // the binary64 path's activations
@@ -197,12 +197,10 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
   __shared__ QatTileRows R;
   const int tid = threadIdx.x;
   const int D = a.D, words = D / 16, quads = D / 256;
-  const int m0 = 2 * tile;
   const int lane = tid & 63, wave = tid >> 6, j = lane & 15, g = lane >> 4;
   const int n_tiles = a.V / 16;
   const int t_lo = (int)((int64_t)blockIdx.x * n_tiles / gridDim.x);
   const int t_hi = (int)((int64_t)(blockIdx.x + 1) * n_tiles / gridDim.x);
-  const int rows_here = a.M - m0 < 2 ? a.M - m0 : 2;
   // Every global access below is a buffer access with no branch around it:
   // codes of tiles past the run or of quads past the width, activations past
   // the rows and logits a lane does not own take an out-of-range offset (zeros, no memory request; stores
@@ -211,10 +209,9 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
   const __amdgpu_buffer_rsrc_t cr =
       __builtin_amdgcn_make_buffer_rsrc((void*)a.words, (short)0, a.V * words * 4, kBufferWord3);
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, (short)0, a.V * 4, kBufferWord3);
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + (int64_t)m0 * D), (short)0,
-                                                                      rows_here * D * 4, kBufferWord3);
-  const __amdgpu_buffer_rsrc_t orr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.out + (int64_t)m0 * a.V), (short)0,
-                                                                       rows_here * a.V * 4, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, a.M * D * 4, kBufferWord3);
+  const __amdgpu_buffer_rsrc_t orr =
+      __builtin_amdgcn_make_buffer_rsrc((void*)a.out, (short)0, a.M * a.V * 4, kBufferWord3);
   // words 16 q + 4 g .. + 3 of vocabulary row n (block 4 q + g in block-major
   // order) and the row's scale
   auto load = [&](int vt, u32x4 (&cw)[kQatMaxSteps / 4], float& sc) __attribute__((always_inline)) {
@@ -297,7 +294,7 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
   __syncthreads();
   bool ok[2];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) ok[q] = m0 + q < a.M && !R.bad[q] && R.sabs[q] < kQatSumBound;
+  for (int q = 0; q < 2; ++q) ok[q] = q < a.M && !R.bad[q] && R.sabs[q] < kQatSumBound;
 
   const bool any_ok = ok[0] || ok[1];
   // the limbs: tile row 8 rr + l, balanced base-256 digits of A (zeros for a
@@ -347,7 +344,7 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
         }
       }
     }
-    // lane (j, g) holds tile rows 4 g .. 4 g + 3: row m0 + g / 2, limbs
+    // lane (j, g) holds tile rows 4 g .. 4 g + 3: row g / 2, limbs
     // 4 (g & 1) .. + 3; the limbs combine in wrapping 64-bit arithmetic (the
     // total is below 2^53 in magnitude, so the wrapped sum is exact)
     uint64_t p = 0;
@@ -377,11 +374,11 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a, in
   // rows the check refused: the binary64 path over this run's vocabulary
   // rows, the activations staged where the operand tile was
   const bool skip[2] = {ok[0], ok[1]};
-  if (!(skip[0] && (skip[1] || m0 + 1 >= a.M))) {
+  if (!(skip[0] && (skip[1] || a.M < 2))) {
     __syncthreads();
-    qat_stage_act<2, kQatTileThreads>(a, m0, L.act);
+    qat_stage_act<2, kQatTileThreads>(a, 0, L.act);
     for (int64_t r = (int64_t)t_lo * 16 + tid; r < (int64_t)t_hi * 16; r += kQatTileThreads)
-      qat_row_binary64<2>(a, m0, skip, L.act, r);
+      qat_row_binary64<2>(a, 0, skip, L.act, r);
   }
 }
 
@@ -729,13 +726,6 @@ __global__ __launch_bounds__(kQatGemmThreads) void qat_gemm_kernel(QatArgs a, in
 
 }  // namespace
 
-// rows of x per pass for width D (the LDS stage holds kQatLdsDoubles)
-int qat_rows_per_pass(int32_t D) {
-  const int r = kQatLdsDoubles / D;
-  return r >= 4 ? 4 : (r >= 2 ? 2 : 1);
-}
-
-
 void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* words, int32_t block_major,
                        const float* scales, int32_t V, double in_scale, double out_scale, float* out,
                        int32_t cu_count, hipStream_t s, LaunchEvents ev) {
@@ -744,7 +734,16 @@ void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* wor
   if (D % 256 == 0 && D <= 2048 && V % 16 == 0 && M <= 2) {
     // one or two rows: one workgroup per compute unit, the codes streamed past
     // eight limb rows (24 us at V 262144, D 1536; qat_gemm_kernel 36)
-    hipExtLaunchKernelGGL(qat_tile_kernel, dim3(cus), dim3(kQatTileThreads), 0, s, ev.start, ev.stop, 0, a, 0);
+    hipExtLaunchKernelGGL(qat_tile_kernel, dim3(cus), dim3(kQatTileThreads), 0, s, ev.start, ev.stop, 0, a);
+    return;
+  }
+  const dim3 grid((unsigned)((V + kQatThreads - 1) / kQatThreads));
+  if (D <= 640 && M <= 2 && (int64_t)V * D * M <= kQatSmall) {
+    // little work: the check and the limbs would take longer (one row of
+    // V 32000, D 320 6 us, qat_gemm_kernel 11; of V 100003, D 576 14 and 16; of
+    // V 32001, D 1088 15 and 13)
+    if (M == 1) hipExtLaunchKernelGGL(qat_lmhead_kernel<1>, grid, dim3(kQatThreads), 0, s, ev.start, ev.stop, 0, a, 0);
+    else hipExtLaunchKernelGGL(qat_lmhead_kernel<2>, grid, dim3(kQatThreads), 0, s, ev.start, ev.stop, 0, a, 0);
     return;
   }
   if (D <= 2048) {
@@ -760,19 +759,10 @@ void launch_qat_lmhead(const float* x, int32_t M, int32_t D, const uint32_t* wor
                           ev.stop, 0, a, groups, runs);
     return;
   }
-  const dim3 grid((unsigned)((V + kQatThreads - 1) / kQatThreads));
-  const int most = qat_rows_per_pass(D);
-  for (int32_t m0 = 0; m0 < M;) {
-    // as many rows of x as the stage holds and remain, in a kernel made for that many
-    const int left = M - m0;
-    const int per = most >= 4 && left >= 4 ? 4 : (most >= 2 && left >= 2 ? 2 : 1);
-    const bool last = m0 + per >= M;
-    hipEvent_t start = m0 == 0 ? ev.start : nullptr, stop = last ? ev.stop : nullptr;
-    if (per == 4) hipExtLaunchKernelGGL(qat_lmhead_kernel<4>, grid, dim3(kQatThreads), 0, s, start, stop, 0, a, m0);
-    else if (per == 2) hipExtLaunchKernelGGL(qat_lmhead_kernel<2>, grid, dim3(kQatThreads), 0, s, start, stop, 0, a, m0);
-    else hipExtLaunchKernelGGL(qat_lmhead_kernel<1>, grid, dim3(kQatThreads), 0, s, start, stop, 0, a, m0);
-    m0 += per;
-  }
+  // wider: a launch per row
+  for (int32_t m = 0; m < M; ++m)
+    hipExtLaunchKernelGGL(qat_lmhead_kernel<1>, grid, dim3(kQatThreads), 0, s, m == 0 ? ev.start : nullptr,
+                          m == M - 1 ? ev.stop : nullptr, 0, a, m);
 }
 
 }  // namespace gs

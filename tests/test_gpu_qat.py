@@ -172,7 +172,7 @@ def test_signed_zero_logits():
         s.close()
 
 
-@pytest.mark.parametrize("V,D,M", [(1000, 64, 1), (1003, 320, 2), (96, 256, 3), (1000, 1536, 16), (2081, 1536, 17),
+@pytest.mark.parametrize("V,D,M", [(1000, 64, 1), (1003, 320, 2), (1003, 704, 1), (1003, 704, 2), (96, 256, 3), (1000, 1536, 16), (2081, 1536, 17),
                                    (515, 1984, 5), (1056, 2048, 9), (300, 2048, 35), (300, 2112, 3)])
 @pytest.mark.parametrize("in_scale", [0.0, 0.03])
 def test_row_groups_bit_exact(V, D, M, in_scale):
