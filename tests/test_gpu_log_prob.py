@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 # one element, less than a 16-byte piece, around a thread's and a part's share,
 # odd and whole multiples; row counts on both sides of one part per row
-@pytest.mark.parametrize("vocab,rows", [(1, 3), (3, 2), (7, 5), (1023, 4), (8193, 33), (40001, 3), (262144, 2),
+@pytest.mark.parametrize("vocab,rows", [(1, 3), (3, 2), (7, 5), (1023, 4), (4096, 5), (8192, 3), (8193, 33), (40001, 3), (262144, 2),
                                         (151643, 1), (4099, 2100)])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_log_prob_rows(vocab, rows, dtype):
