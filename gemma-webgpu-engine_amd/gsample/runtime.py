@@ -240,19 +240,11 @@ class SampleOutput:
     flags: np.ndarray
 
 
-def full_draw_rows(cfg: np.ndarray) -> bool:
-    """Whether any packed row config may take a full-vocabulary draw
-    (temperature > 0, topK 0, topP 1, no min-p or typical-p, no mask): the
-    batch hint GS_BATCH_FULL_DRAWS (include/gsample.h)."""
-    c = np.asarray(cfg).reshape(-1)
-    return bool(np.any((c["temperature"] > 0) & (c["top_k"] <= 0) & (c["top_p"] >= 1) & ~(c["min_p"] > 0)
-                       & (c["typical_p"] >= 1) & (c["mask_slot"] < 0)))
-
-
 def batch_hints(cfg: np.ndarray, vocab: int) -> int:
-    """The hints of a batch of packed row configs: GS_BATCH_FULL_DRAWS as
-    full_draw_rows says, GS_BATCH_TYPICAL when a row may take typical-p over
-    the whole vocabulary (topK 0 or all, topP 1, no min-p, no mask)."""
+    """The hints of a batch of packed row configs: GS_BATCH_FULL_DRAWS when a
+    row may take a full-vocabulary draw (temperature > 0, topK 0, topP 1, no
+    min-p or typical-p, no mask), GS_BATCH_TYPICAL when one may take typical-p
+    over the whole vocabulary (topK 0 or all, topP 1, no min-p, no mask)."""
     c = np.asarray(cfg).reshape(-1)
     if c.size == 1 and c["top_p"][0] < 1:  # an interactive row's usual options, settled by one field
         return 0
@@ -263,6 +255,13 @@ def batch_hints(cfg: np.ndarray, vocab: int) -> int:
     full = bool(np.any(free & ~typical & (top_k <= 0)))
     spread = bool(np.any(free & typical & ((top_k <= 0) | (top_k >= vocab))))
     return (GS_BATCH_FULL_DRAWS if full else 0) | (GS_BATCH_TYPICAL if spread else 0)
+
+
+def full_draw_rows(cfg: np.ndarray) -> bool:
+    """Whether any packed row config may take a full-vocabulary draw
+    (temperature > 0, topK 0, topP 1, no min-p or typical-p, no mask): the
+    batch hint GS_BATCH_FULL_DRAWS (include/gsample.h)."""
+    return bool(batch_hints(cfg, np.iinfo(np.int32).max) & GS_BATCH_FULL_DRAWS)
 
 
 def _csr(lists: Optional[Sequence[Sequence[int]]], rows: int):
