@@ -14,8 +14,11 @@
 //     row blocks of a slab of W one after another). At D 2048, V 262144:
 //     M 128 takes 220 us (5.5 TB/s), M 256 350, M 512 665 (830 TFLOP/s);
 //     the resident kernel, launched once per 64 rows, took 399, 793 and 1582.
-//     At M 12, D 3840, V 151643 217 us (5.4 TB/s) against 272 for a kernel
-//     that held the rows of W it multiplied in registers.
+//     At M 12, D 3840, V 151643 226 us (5.2 TB/s) against 281 for a kernel
+//     that held the rows of W it multiplied in registers; that one was the
+//     faster of the two up to D 704 with 33 to 64 rows of such a vocabulary
+//     (M 64, V 151643: D 512 37 us against 42, D 704 46 against 50), where a
+//     workgroup's few K blocks do not hide its start and its end.
 // What bounds the GEMM: memory up to about 160 rows; past that the operand
 // traffic of the tiles (12 TB/s from the L2s at M 512), the matrix cores 42%
 // busy. The totals of the ranges take the registers that a larger tile would.

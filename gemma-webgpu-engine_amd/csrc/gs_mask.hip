@@ -1,8 +1,9 @@
 // Constraint masker and raw-logit log-probability.
 //
-// build_masks_kernel: legalTokenIds (src/runtime/constraints.ts:56-92) for a
-// byte-level DFA, as a 262144-bit mask per requested state. The reference
-// walks a token-byte trie depth-first; here every token walks its own bytes
+// walk_masks_kernel and build_masks_kernel: legalTokenIds
+// (src/runtime/constraints.ts:56-92) for a byte-level DFA, as a 262144-bit
+// mask per requested state. The reference walks a token-byte trie
+// depth-first; here every token walks its own bytes
 // (the vocab is a CSR of token byte strings), one token per lane, against a
 // next-state table whose entries already fold in viability
 // (src/runtime/constraints.ts:253-265, 300-322): next'[s][b] = -1 unless the

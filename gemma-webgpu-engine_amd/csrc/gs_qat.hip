@@ -20,19 +20,21 @@
 // HBM: V * D / 4 bytes of codes (96 MiB at V 262144, D 1536) + 4 V of scales
 // + 4 M V of logits per call; the activations (M x D) are staged in LDS as
 // binary64. Work: one bit-field extract, one conversion and one fused
-// multiply-add per weight and row of x.
+// multiply-add per weight and row of x. qat_lmhead_kernel does so for widths
+// past 2048 and for little work (launch_qat_lmhead).
 //
-// Exact integer path (widths a multiple of 256 up to 2048, V a multiple of
-// 16). Every activation a_k is a binary32 value, an integer multiple of its
+// Exact integer path (widths up to 2048). Every activation a_k is a binary32 value, an integer multiple of its
 // granule 2^g_k; with E the smallest granule of a row (nonzero a_k), every
 // product (code - 2) a_k and every partial sum is an integer multiple of 2^E
 // no larger than 2 sum |a_k|. When that bound is below 2^(E + 53), no partial
 // sum rounds: the sequential binary64 sum is the exact sum, and so is
 //   2^E (sum_k code_k A_k - 2 sum_k A_k),   A_k = a_k / 2^E (integers).
-// qat_tile_kernel checks the bound per row of x, writes A_k as 7 balanced
-// base-256 digits (int8 limbs), multiplies the codes (0..3, int8) by the
-// limbs on v_mfma_i32_16x16x64_i8 (exact int32 sums), combines the limbs in
-// wrapping 64-bit arithmetic (exact: the total fits in 53 bits) and applies
+// qat_tile_kernel (one or two rows, widths a multiple of 256, V a multiple of
+// 16) and qat_gemm_kernel (groups of 16 rows, any width and V) check the
+// bound per row of x, write A_k as up to 7 balanced
+// base-256 digits (int8 limbs), multiply the codes (0..3, int8) by the
+// limbs on v_mfma_i32_16x16x64_i8 (exact int32 sums), combine the limbs in
+// wrapping 64-bit arithmetic (exact: the total fits in 53 bits) and apply
 // the same epilogue, so the logits equal the binary64 path's bit for bit.
 // Rows that fail the bound (a huge exponent range, subnormals, non-finite
 // values) take the binary64 path in the same launch.
@@ -394,8 +396,8 @@ __global__ __launch_bounds__(kQatTileThreads) void qat_tile_kernel(QatArgs a) {
 // limbs are multiplied as the group's largest |A_k| has: 5 for activations of
 // an input SRQ, 5 or 6 for normal ones. The groups of one run are on one XCD,
 // so its codes come from HBM once. V 262144, D 1536, input SRQ: 3 rows
-// 40 us, 16 rows 59, 32 rows 81, 48 rows 106 (714 by qat_tile_kernel, a launch
-// per two rows), 64 rows 129; D 2048 without SRQ, 48 rows (eight at a time)
+// 40 us, 16 rows 59, 32 rows 81, 48 rows 106 (714 in launches of
+// qat_tile_kernel for two rows each), 64 rows 129; D 2048 without SRQ, 48 rows (eight at a time)
 // 194. Bound by the limbs read from LDS and the matrix cores (38 us each at
 // 48 rows); the check and the limbs take about 10 us a workgroup.
 constexpr int kQatGemmThreads = 512;

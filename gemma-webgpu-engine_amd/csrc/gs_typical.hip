@@ -12,18 +12,19 @@
 //
 // A decision that the reference's own rounding could turn (its sequential
 // sums move by V 2^-53 relative) is left to the exact replay: a sum within
-// `margin` of its threshold, two different logits whose surprises differ by
-// less than the entropy's error at the cut, two whose probabilities could
-// round either way at the draw. The bins' sums vary in their last bits with
+// `margin` of its threshold, a logit other than the cut's whose surprise lies
+// within the entropy's error of it, one other than the drawn whose
+// probability could round either way. So are lists of more than kTypCap
+// items: more equal logits than that at the cut or in the drawn bin. The bins' sums vary in their last bits with
 // the order of the LDS atomics: no decision rests on those, only, within
 // 1e-15 of the margin's own edge, whether the replay takes it.
 //
 // Bound by the exponential pass on one CU (about 30 binary64 operations a
-// logit); more workgroups a row would need a launch for each of the four
-// steps. Whole calls: 24 rows of 151643 f32 logits 112 us (125 before the
-// gathers skipped waves without an item by a comparison in binary32), 256 rows
-// of 262144 240 us; the replays, with three sorts and five one-lane sums a row, took
-// 27.3 and 29.9 ms. Probabilities are within 4e-16 of 64-bit ones (2.4e-14).
+// logit); spreading a row over workgroups would take a launch, about 5 us, for
+// each of the four steps. Whole calls: 24 rows of 151643 f32 logits 113 us (125
+// before the gathers skipped waves without an item by a comparison in
+// binary32), 256 rows of 262144 240 us; the replays, with three sorts and five
+// one-lane sums a row, took 27.3 and 29.9 ms. Probabilities are within 4e-16 of 64-bit ones (2.4e-14).
 #include "gs_exact_row.h"
 #include "gs_exp2.h"
 
