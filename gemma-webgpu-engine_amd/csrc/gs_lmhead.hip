@@ -9,16 +9,13 @@
 // whichever kernel and batch it comes from (and about half the rounding error
 // of one chain over K: 1.1e-7 against 2.0e-7 relative at D 2048).
 //   * up to 64 rows, widths up to 2048: lmhead_resident_kernel, H in registers;
-//   * anything else: lmhead_gemm_kernel, tiles of 128 vocabulary rows by up to
-//     128 rows of H. W is read from HBM once whatever M is (an XCD takes the
+//   * anything else: lmhead_gemm_kernel, tiles of 128 vocabulary rows (64 for
+//     narrow heads of odd vocabularies, launch_lmhead) by up to 128 rows of H. W is read from HBM once whatever M is (an XCD takes the
 //     row blocks of a slab of W one after another). At D 2048, V 262144:
 //     M 128 takes 220 us (5.5 TB/s), M 256 350, M 512 665 (830 TFLOP/s);
 //     the resident kernel, launched once per 64 rows, took 399, 793 and 1582.
 //     At M 12, D 3840, V 151643 226 us (5.2 TB/s) against 281 for a kernel
-//     that held the rows of W it multiplied in registers; that one was the
-//     faster of the two up to D 704 with 33 to 64 rows of such a vocabulary
-//     (M 64, V 151643: D 512 37 us against 42, D 704 46 against 50), where a
-//     workgroup's few K blocks do not hide its start and its end.
+//     that held the rows of W it multiplied in registers.
 // What bounds the GEMM: memory up to about 160 rows; past that the operand
 // traffic of the tiles (12 TB/s from the L2s at M 512), the matrix cores 42%
 // busy. The totals of the ranges take the registers that a larger tile would.
@@ -83,10 +80,8 @@ __device__ __forceinline__ void lmhead_cap(float (&x)[kN], float cap, float r) {
 }
 
 constexpr int kGemmThreads = 256;  // 2 x 2 waves over (V, M)
-constexpr int kGemmV = 128;        // vocabulary rows per workgroup
 constexpr int kGemmK = 64;         // K block: one 128-byte line of every row
 constexpr int kGemmChunks = 8;     // K ranges summed one by one, as the resident kernel's waves do
-constexpr int kGemmStride = kGemmV + 4;  // LDS floats per staged output row
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -106,10 +101,10 @@ __device__ __forceinline__ void gemm_fetch(Rsrc r, char* lds, const uint32_t (&o
 }
 
 // The running tiles into the totals, at the end of a range of K.
-template <int kMT>
-__device__ __forceinline__ void gemm_flush(f32x4 (&acc)[4][kMT], f32x4 (&total)[4][kMT]) {
+template <int kVT, int kMT>
+__device__ __forceinline__ void gemm_flush(f32x4 (&acc)[kVT][kMT], f32x4 (&total)[kVT][kMT]) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int a = 0; a < kVT; ++a) {
 #pragma unroll
     for (int b = 0; b < kMT; ++b) {
       total[a][b] += acc[a][b];
@@ -119,52 +114,53 @@ __device__ __forceinline__ void gemm_flush(f32x4 (&acc)[4][kMT], f32x4 (&total)[
 }
 
 // One K block: the next fetches go out, then two K-32 steps of this wave's
-// 4 x kMT tiles; a range ends (uniform) after the second step or, with
+// kVT x kMT tiles; a range ends (uniform) after the second step or, with
 // kHalf, also after the first. The buffers are distinct objects, so the
 // compiler's own waits before the reads cover nothing that is still being
 // fetched.
-template <int kMT, bool kHalf, typename Rsrc>
+template <int kVT, int kMT, bool kHalf, typename Rsrc>
 __device__ __forceinline__ void gemm_block(const char* __restrict__ w, const char* __restrict__ h,
                                            char* __restrict__ w_next, char* __restrict__ h_next,
                                            Rsrc wr, Rsrc hr,
-                                           const uint32_t (&w_off)[4], const uint32_t (&h_off)[kMT], uint32_t w_k,
+                                           const uint32_t (&w_off)[kVT], const uint32_t (&h_off)[kMT], uint32_t w_k,
                                            uint32_t h_k, const uint32_t (&pos)[2], bool half_flush, bool flush,
-                                           f32x4 (&acc)[4][kMT], f32x4 (&total)[4][kMT]) {
+                                           f32x4 (&acc)[kVT][kMT], f32x4 (&total)[kVT][kMT]) {
   gemm_fetch<kMT>(hr, h_next, h_off, h_k);
-  asm volatile("" ::: "memory");  // W's fetches stay the last four issued
-  gemm_fetch<4>(wr, w_next, w_off, w_k);
-  bf16x8 wf[2][4], hf[2][kMT];
+  asm volatile("" ::: "memory");  // W's fetches stay the last kVT issued
+  gemm_fetch<kVT>(wr, w_next, w_off, w_k);
+  bf16x8 wf[2][kVT], hf[2][kMT];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) wf[s][a] = *(const bf16x8*)(w + pos[s] + 2048 * a);
+    for (int a = 0; a < kVT; ++a) wf[s][a] = *(const bf16x8*)(w + pos[s] + 2048 * a);
 #pragma unroll
     for (int b = 0; b < kMT; ++b) hf[s][b] = *(const bf16x8*)(h + pos[s] + 2048 * b);
   }
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < kVT; ++a) {
 #pragma unroll
       for (int b = 0; b < kMT; ++b)
         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][a], hf[s][b], acc[a][b], 0, 0, 0);
     }
-    if (kHalf && s == 0 && half_flush) gemm_flush<kMT>(acc, total);
+    if (kHalf && s == 0 && half_flush) gemm_flush<kVT, kMT>(acc, total);
   }
-  if (flush) gemm_flush<kMT>(acc, total);
+  if (flush) gemm_flush<kVT, kMT>(acc, total);
 }
 
-// kMT: 16-row tiles of H per wave (32 kMT rows of H per workgroup). kHalf:
-// the resident kernel's ranges at widths off 512, which may end within a K
-// block; where that kernel never runs they end with blocks (the flush between
-// a block's steps costs up to 3%, and ranges of whole blocks would cost the
-// resident kernel up to 6% there: V 32000, D 576, one row 15.9 us | 15.0).
-template <int kMT, bool kHalf>
-__global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint16_t* __restrict__ H,
-                                                                      const uint16_t* __restrict__ W, int M, int D,
-                                                                      int V, int m_blocks, int wide, float cap,
-                                                                      float* __restrict__ out) {
-  constexpr int kRows = 32 * kMT;
+// kVT, kMT: 16-row tiles of W and H per wave (32 kVT vocabulary rows and
+// 32 kMT rows of H per workgroup). kHalf: the resident kernel's ranges at
+// widths off 512, which may end within a K block; where that kernel never runs
+// they end with blocks (the flush between a block's steps costs up to 3%, and
+// ranges of whole blocks would cost the resident kernel up to 6% there:
+// V 32000, D 576, one row 15.9 us | 15.0).
+template <int kVT, int kMT, bool kHalf>
+__global__ __launch_bounds__(kGemmThreads, kVT == 2 ? 4 : 2) void lmhead_gemm_kernel(
+    const uint16_t* __restrict__ H, const uint16_t* __restrict__ W, int M, int D, int V, int m_blocks, int wide,
+    float cap, float* __restrict__ out) {
+  constexpr int kGemmV = 32 * kVT, kRows = 32 * kMT;
+  constexpr int kGemmStride = kGemmV + 4;  // LDS floats per staged output row
   constexpr int kWBytes = kGemmV * kGemmK * 2, kHBytes = kRows * kGemmK * 2;
   // three blocks of W and two of H; the staged outputs take their place
   __shared__ __attribute__((aligned(16))) char lds[3 * kWBytes + 2 * kHBytes];
@@ -186,23 +182,23 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
       __builtin_amdgcn_make_buffer_rsrc((void*)(W + (size_t)v0 * D), (short)0, v_rows * D * 2, kBufferWord3);
   const __amdgpu_buffer_rsrc_t hr =
       __builtin_amdgcn_make_buffer_rsrc((void*)(H + (size_t)m0 * D), (short)0, m_rows * D * 2, kBufferWord3);
-  // this wave fetches rows 32 wave .. + 31 of W's block and 8 kMT wave .. of H's
+  // this wave fetches rows 8 kVT wave .. of W's block and 8 kMT wave .. of H's
   const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 16;
-  uint32_t w_off[4], h_off[kMT];
+  uint32_t w_off[kVT], h_off[kMT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w_off[i] = (uint32_t)((32 * wave + 8 * i + lr) * D * 2 + lc);
+  for (int i = 0; i < kVT; ++i) w_off[i] = (uint32_t)((8 * kVT * wave + 8 * i + lr) * D * 2 + lc);
 #pragma unroll
   for (int i = 0; i < kMT; ++i) h_off[i] = (uint32_t)((8 * kMT * wave + 8 * i + lr) * D * 2 + lc);
-  const int w_dst = 32 * wave * 128, h_dst = 8 * kMT * wave * 128;
+  const int w_dst = 8 * kVT * wave * 128, h_dst = 8 * kMT * wave * 128;
   // operand reads: lane (j, g) holds k = 32 s + 8 g .. + 7 of row j of a tile
   uint32_t pos[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) pos[s] = (uint32_t)(j * 128 + (((4 * s + g) ^ (j & 7)) * 16));
-  const int w_src = 64 * wv * 128, h_src = 16 * kMT * wm * 128;
+  const int w_src = 16 * kVT * wv * 128, h_src = 16 * kMT * wm * 128;
 
-  f32x4 acc[4][kMT], total[4][kMT];
+  f32x4 acc[kVT][kMT], total[kVT][kMT];
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
+  for (int a = 0; a < kVT; ++a) {
 #pragma unroll
     for (int b = 0; b < kMT; ++b) {
       acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -227,18 +223,19 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
   auto block = [&](int kb, char* w, char* h, char* wn, char* hn) __attribute__((always_inline)) {
     // block kb's rows have landed for every wave (W's block kb + 1, fetched
     // after them, may still be under way), and every wave has read block kb - 1
-    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (kVT == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const bool half_flush = kHalf && 2 * kb + 1 == bound;
     if (half_flush) next_bound();
     const bool flush = 2 * kb + 2 == bound;
     if (flush) next_bound();
-    gemm_block<kMT, kHalf>(w + w_src, h + h_src, wn + w_dst, hn + h_dst, wr, hr, w_off, h_off, at(kb + 2), at(kb + 1),
+    gemm_block<kVT, kMT, kHalf>(w + w_src, h + h_src, wn + w_dst, hn + h_dst, wr, hr, w_off, h_off, at(kb + 2), at(kb + 1),
                            pos, half_flush, flush, acc, total);
   };
-  gemm_fetch<4>(wr, sw0 + w_dst, w_off, at(0));
+  gemm_fetch<kVT>(wr, sw0 + w_dst, w_off, at(0));
   gemm_fetch<kMT>(hr, sh0 + h_dst, h_off, at(0));
   asm volatile("" ::: "memory");
-  gemm_fetch<4>(wr, sw1 + w_dst, w_off, at(1));
+  gemm_fetch<kVT>(wr, sw1 + w_dst, w_off, at(1));
   // blocks past the last are fetched as the last one again, and not read
   for (int kb = 0;; kb += 6) {
     block(kb, sw0, sh0, sw2, sh1);
@@ -265,10 +262,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void lmhead_gemm_kernel(const uint
 #pragma unroll
   for (int b = 0; b < kMT; ++b) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < kVT; ++a) {
       float x[4] = {total[a][b][0], total[a][b][1], total[a][b][2], total[a][b][3]};
       if (cap > 0.0f) lmhead_cap<4>(x, cap, rcap);
-      *(f32x4*)&stage[(16 * (kMT * wm + b) + j) * kGemmStride + 64 * wv + 16 * a + 4 * g] = f32x4{x[0], x[1], x[2], x[3]};
+      *(f32x4*)&stage[(16 * (kMT * wm + b) + j) * kGemmStride + 16 * kVT * wv + 16 * a + 4 * g] = f32x4{x[0], x[1], x[2], x[3]};
     }
   }
   __syncthreads();
@@ -478,23 +475,35 @@ void launch_lmhead(const uint16_t* hidden, const uint16_t* weight, int32_t m, in
   // blocks of at most 128 rows of H, the rows spread evenly over them
   const int m_blocks = (m + 127) / 128;
   const int tiles = ((m + m_blocks - 1) / m_blocks + 31) / 32;  // per wave: 1 .. 4
-  const int v_tiles = (vocab + kGemmV - 1) / kGemmV;
+  const int half = resident && width % 512 != 0;
+  // Tiles of 64 vocabulary rows, four workgroups a compute unit, where a row
+  // block is small, the larger tiles would take more than one round of
+  // workgroups and the weights about fit the last-level cache: the start and
+  // end of a workgroup weigh there. 64 rows of V 151643, D 704 46 us (50 in
+  // tiles of 128), V 200003, D 512 51 (56), V 262143, D 512 57 (67), but V 50257,
+  // D 704 19 (17) and V 262143, D 576 79 (73), D 3840 436 (361).
+  const int cus = cu_count > 0 ? cu_count : 256;
+  const bool narrow = tiles <= 2 && !half && (vocab + 127) / 128 > 2 * cus && (int64_t)vocab * width <= 145000000;
+  const int v_rows = narrow ? 64 : 128;
+  const int v_tiles = (vocab + v_rows - 1) / v_rows;
   const dim3 grid((unsigned)((v_tiles + 7) / 8 * 8 * m_blocks)), block(kGemmThreads);
   const int wide = vocab % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  switch (resident && width % 512 != 0 ? -tiles : tiles) {
-#define GS_GEMM_CASE(n, k, half)                                                                                       \
+  switch (narrow ? 20 + tiles : (half ? 10 + tiles : tiles)) {
+#define GS_GEMM_CASE(n, vt, k, half)                                                                                   \
   case n:                                                                                                              \
-    hipExtLaunchKernelGGL((lmhead_gemm_kernel<k, half>), grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight, m,   \
-                          width, vocab, m_blocks, wide, softcap, out);                                                 \
+    hipExtLaunchKernelGGL((lmhead_gemm_kernel<vt, k, half>), grid, block, 0, s, ev.start, ev.stop, 0, hidden, weight,  \
+                          m, width, vocab, m_blocks, wide, softcap, out);                                              \
     break;
-    GS_GEMM_CASE(1, 1, false)
-    GS_GEMM_CASE(2, 2, false)
-    GS_GEMM_CASE(3, 3, false)
-    GS_GEMM_CASE(4, 4, false)
-    GS_GEMM_CASE(-1, 1, true)
-    GS_GEMM_CASE(-2, 2, true)
-    GS_GEMM_CASE(-3, 3, true)
-    GS_GEMM_CASE(-4, 4, true)
+    GS_GEMM_CASE(1, 4, 1, false)
+    GS_GEMM_CASE(2, 4, 2, false)
+    GS_GEMM_CASE(3, 4, 3, false)
+    GS_GEMM_CASE(4, 4, 4, false)
+    GS_GEMM_CASE(11, 4, 1, true)
+    GS_GEMM_CASE(12, 4, 2, true)
+    GS_GEMM_CASE(13, 4, 3, true)
+    GS_GEMM_CASE(14, 4, 4, true)
+    GS_GEMM_CASE(21, 2, 1, false)
+    GS_GEMM_CASE(22, 2, 2, false)
 #undef GS_GEMM_CASE
   }
 }

@@ -163,6 +163,9 @@ def test_lmhead_shapes_match_f64(vocab, width, m):
     (1028, 192, 70, 0),    # ranges of one step, two in a K block
     (1027, 576, 100, 0),   # no resident kernel at this vocabulary: ranges of whole blocks
     (127, 2048, 33, 0),    # less than one slab, odd rows
+    (66003, 256, 17, 0),   # slabs of 64: one- and two-tile row blocks, four K blocks over eight ranges,
+    (66003, 576, 40, 0),   # nine, and ranges started in turn; the last slab partial
+    (66067, 512, 64, 0),
     (2049, 3840, 1, 0),    # wide, odd, one row
 ])
 def test_lmhead_gemm_edges(vocab, width, m, shift):
@@ -193,5 +196,9 @@ def test_lmhead_gemm_edges(vocab, width, m, shift):
             if vocab % 4 == 0 and width <= 2048 and (m > 64 or shift):
                 alone = s.lmhead(hidden[:64].contiguous(), weight, softcap_value=cap)
                 assert torch.equal(alone, out[:min(m, 64)])
+            if vocab > 65536:  # the larger slabs of a larger batch: the same bits
+                more = s.lmhead(torch.cat([hidden, hidden, hidden, hidden])[:100].contiguous(), weight,
+                                softcap_value=cap)
+                assert torch.equal(more[:m], out[:m])
     finally:
         s.close()
