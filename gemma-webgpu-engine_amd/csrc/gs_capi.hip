@@ -826,10 +826,11 @@ int gs_check_exp2(gs_context* ctx, float lo, float hi, double* max_rel_err, floa
   return GS_OK;
 }
 
-// live_share from the vocabulary's first bytes and the DFA (both set).
+// live_share from the vocabulary's first bytes and the DFA, once both are set
+// (a call that failed may have left either half replaced: zeros then).
 static void count_live(gs_context* ctx) {
   ctx->live_share.assign(ctx->next.size() / 256, 0.0);
-  if (ctx->first_bytes.empty()) return;
+  if (ctx->first_bytes.empty() || ctx->viable.size() != ctx->live_share.size()) return;
   for (size_t s = 0; s < ctx->live_share.size(); ++s) {
     int64_t live = 0;
     for (int c = 0; c < 256; ++c) {
